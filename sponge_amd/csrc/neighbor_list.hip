@@ -468,8 +468,8 @@ __device__ __forceinline__ void nl_search_cells_body(int sa_block,
     // than the list radius from the box: a pair within the list radius has
     // these images at its minimum-image displacement (see the sweep below),
     // so no partner is lost; the margin covers the rounding of both sides.
+    // (without these images every candidate joins)
     auto keeps = [&](int q) -> bool {
-        if (!shift) return true;
         const float4 v = spos[q];
         const float3 w = near_image(make_float3(v.x, v.y, v.z), C, c, r);
         const float dx = fmaxf(0.f, fmaxf(blo.x - w.x, w.x - bhi.x));
@@ -478,13 +478,26 @@ __device__ __forceinline__ void nl_search_cells_body(int sa_block,
         const float m = fmaxf(mrow, fmaxf(fabsf(v.x), fmaxf(fabsf(v.y), fabsf(v.z))));
         return fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < thr + search_margin(m, Lmax, thr);
     };
-    // kept atoms per run, then their offsets, then the stream itself (the
-    // second pass repeats the test: its loads hit the caches)
+    // The test is made once per candidate: its outcome is kept as a bit, 64
+    // candidates of a run to a word, and the counts, the offsets and the stream
+    // all come from these words, so that they agree whatever the arithmetic of
+    // the test rounds to.  The words lie in the chunk's buffer, which is staged
+    // later; run k has the words from (r_off[k] >> 6) + k on.
+    unsigned long long* bits = reinterpret_cast<unsigned long long*>(cand);
+    static_assert(sizeof(unsigned long long) * ((65535 >> 6) + kMaxRanges + 1) <= sizeof(cand),
+                  "words of the longest stencil");
     for (int k = wave; k < nr; k += nwave) {
         const int f = r_first[k], len = r_off[k + 1] - r_off[k];
-        int kept = 0;
-        for (int u = 0; u < len; u += kWave)
-            kept += (int)__popcll(__ballot(u + lane < len && keeps(f + min(u + lane, len - 1))));
+        int kept = len;
+        if (shift) {
+            kept = 0;
+            for (int u = 0; u < len; u += kWave) {
+                const unsigned long long m =
+                    __ballot(u + lane < len && keeps(f + min(u + lane, len - 1)));
+                if (lane == 0) bits[(r_off[k] >> 6) + k + (u >> 6)] = m;
+                kept += (int)__popcll(m);
+            }
+        }
         if (lane == 0) r_keep[k + 1] = kept;
     }
     __syncthreads();
@@ -506,10 +519,13 @@ __device__ __forceinline__ void nl_search_cells_body(int sa_block,
         const int f = r_first[k], len = r_off[k + 1] - r_off[k];
         int at = r_keep[k];
         for (int u = 0; u < len; u += kWave) {
-            const bool ok = u + lane < len && keeps(f + min(u + lane, len - 1));
-            const unsigned long long m = __ballot(ok);
-            if (ok) strm[at + lanes_below(m)] = f + u + lane;
-            at += (int)__popcll(m);
+            if (shift) {
+                const unsigned long long m = bits[(r_off[k] >> 6) + k + (u >> 6)];
+                if (m >> lane & 1) strm[at + lanes_below(m)] = f + u + lane;
+                at += (int)__popcll(m);
+            } else if (u + lane < len) {
+                strm[at + u + lane] = f + u + lane;
+            }
         }
     }
     const int rows = a1 - a0;
