@@ -74,6 +74,7 @@ SIGNATURES = {
     "sponge_nl_atom_group": (_I, [_P, C.POINTER(_P)]),
     "sponge_nl_atom_group_address": (_I, [_P, C.POINTER(_P)]),
     "sponge_nl_info": (_I, [_P, C.POINTER(C.c_longlong), C.POINTER(_I)]),
+    "sponge_nl_stream_info": (_I, [_P, C.POINTER(_I), C.POINTER(_I)]),
     "sponge_nl_rebuild_count": (_I, [_P, C.POINTER(C.c_longlong)]),
     "sponge_nl_clear": (_I, [_P]),
     "sponge_lj_initial": (_I, [C.POINTER(_P), _I, _I, _FP, _FP, C.POINTER(_I), _F, _P]),
@@ -293,6 +294,13 @@ class NeighborList:
         d = (C.c_int * 3)()
         _check(self.lib.sponge_nl_info(self.h, C.byref(n), d), "sponge_nl_info")
         return n.value, tuple(d)
+
+    def stream_info(self):
+        """(longest candidate stream, entries of a stream kept on chip)."""
+        longest, staged = C.c_int(), C.c_int()
+        _check(self.lib.sponge_nl_stream_info(self.h, C.byref(longest), C.byref(staged)),
+               "sponge_nl_stream_info")
+        return longest.value, staged.value
 
     def clear(self):
         if self.h:

@@ -29,7 +29,7 @@ struct sponge_nl {
     hipStream_t stream = nullptr;
 
     int* d_need = nullptr;        // rebuild flag of this step
-    int* d_flags = nullptr;       // sticky overflow flags
+    int* d_flags = nullptr;       // [0] sticky overflow flags, [1] longest stream beyond the stage
     unsigned long long* d_rebuilds = nullptr;  // number of list builds
     int* d_cell_count = nullptr;  // [G]
     int* d_ref_count = nullptr;   // [G] atoms per cell of edge grid_length, where width differs from it
@@ -54,6 +54,7 @@ struct sponge_nl {
     int* d_slen = nullptr;        // [G] its length
     unsigned long long* d_sfill = nullptr;  // entries of d_stream handed out in this build
     int stream_mean = 0;          // expected stream length of a cell at the mean density
+    int stream_seen = 0;          // stage for the longest stream found, where that was beyond it
     int* d_exp_serial = nullptr;  // reference-format export storage (lazy)
     int* d_exp_count = nullptr;
     sa_atom_group* d_atom_group = nullptr;
@@ -176,6 +177,9 @@ __device__ __forceinline__ void stage_stream(const int* __restrict__ strm, int l
 // `reserve` further bytes, at most `want`, a multiple of 64.
 int stage_entries(size_t bytes_per_entry, int want, size_t reserve = 0);
 
+// most entries of a candidate stream that the pair kernels stage in LDS
+constexpr int kPairStage = 3584;
+
 // Workgroup size and LDS of a launch of one workgroup per cell that stages the
 // cell's candidate stream (bytes per entry and of the tables beside it; at
 // most `most` entries): see its definition.
@@ -186,6 +190,16 @@ struct PairLaunch {
     size_t lds = 0;
 };
 PairLaunch pair_launch(const sponge_nl* nl, size_t bytes_per_entry, size_t tables, int most);
+
+// Entries of a candidate stream that these launches stage, where LDS has room:
+// a fifth more than the mean expected from the box, or the longest stream that
+// a build reported with a sixteenth to spare (a stream outside the stage costs
+// its cell's rows two dependent memory reads per entry; a liquid slab in a box
+// twice as long has streams of twice the mean).  Builds report streams beyond the
+// stage (d_flags[1]); the host reads that after the first build and at every
+// overflow check and hands it to nl_streams_seen (true: the stage has grown).
+int nl_stream_stage(const sponge_nl* nl);
+bool nl_streams_seen(sponge_nl* nl, int longest);
 
 // Lower and upper faces of cell i of n on an axis of length L (the last cell
 // ends at the box)
@@ -287,7 +301,9 @@ int md_state_arrays(sponge_md* m, float** crd, float** charge);
 int nl_set_prune(sponge_nl* nl, float delta);
 
 // the list's sticky overflow flags, read (synchronising) and cleared
-int nl_take_flags(sponge_nl* nl, int* flags);
+// (longer, nullable: a stream beyond the stage was found; the pair kernels'
+// launches are larger from here on)
+int nl_take_flags(sponge_nl* nl, int* flags, bool* longer = nullptr);
 // Check_Overflow's recovery: *nl replaced by a fresh list with 1.1x the
 // limits named by flags (the caller rebuilds anything that held the old one)
 int nl_reinitialize(sponge_nl** nl, int flags);

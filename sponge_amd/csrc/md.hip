@@ -97,7 +97,7 @@ struct sponge_md {
     // does not exist
     int* d_sx_start = nullptr;  // [N + 1]
     int* d_sx_list = nullptr;
-    int nl_generation = 0;  // bumped when an overflow re-initialises the list
+    int nl_generation = 0;  // bumped when recorded steps no longer hold (the list or its stage is a new one)
     float prune_delta = SPONGE_AMD_MD_LIST_PRUNE_DELTA;  // inner-row buffer of the pair kernel
     int overflow_flags = 0;  // every overflow flag seen by the driver's checks
 };
@@ -689,8 +689,15 @@ int md_check_overflow(sponge_md* m, long long first, long long last) {
     const int iv = m->nl->opt.check_overflow_interval;
     if (iv <= 0 || (last + 1) / iv * iv < first + 1) return 0;
     int flags = 0;
-    int rc = nl_take_flags(m->nl, &flags);
-    if (rc || !flags) return rc;
+    bool longer = false;
+    int rc = nl_take_flags(m->nl, &flags, &longer);
+    if (rc) return rc;
+    if (longer) {
+        // captured and recorded steps hold the pair kernel's former stage
+        drop_graphs(m);
+        m->nl_generation++;
+    }
+    if (!flags) return 0;
     m->overflow_flags |= flags;
     if ((flags & SPONGE_AMD_NL_STREAM_OVERFLOW) || m->nl->opt.throw_error_when_overflow)
         return SPONGE_AMD_ERROR_OVERFLOW;

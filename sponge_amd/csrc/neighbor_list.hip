@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <numeric>
 #include <type_traits>
 #include <vector>
 
@@ -43,38 +44,52 @@ int sa::stage_entries(size_t bytes_per_entry, int want, size_t reserve) {
 // The pair kernels run a workgroup per cell (or `split` of them), a wavefront
 // per row, and hide their list and LDS latencies behind 8 wavefronts per SIMD
 // (32 per CU).  The LDS stage is sized for a stream a fifth longer than the
-// mean; a CU's 160 KiB then hold up to `fit` workgroups of 32 / fit
-// wavefronts.  Streams beyond the stage (a region a fifth denser than the
-// mean) are read from HBM.
+// mean, or for the longest stream known where that is longer (see
+// nl_stream_stage); a CU's 160 KiB then hold up to `fit` workgroups of 32 / fit
+// wavefronts.  Streams beyond the stage are read from HBM.
 // The workgroup size and the split are chosen by a count of cycles: the chip
 // works the workgroups off in whole rounds of 256 x fit, a workgroup costs its
 // staging and its rounds of rows, and a row costs its issue cycles times the
 // wavefronts that share a SIMD (2,300 at 700 entries), or its own latency
 // where those are few.  So 4,096 cells take 8 wavefronts (23 rows in 3
 // rounds), 1,287 cells 10 (a round of 1,024 workgroups and a quarter would
-// idle most of the chip), and 125 cells two workgroups each.
+// idle most of the chip), and 125 cells two workgroups each.  Where streams
+// `dense` times the mean are known (a liquid in a part of the box), the count
+// is that of a part of the cells with so many times the rows.
 // Launches recorded for the batched driver share one size.
+static int round64(int n) { return (n + 63) & ~63; }
+
+int sa::nl_stream_stage(const sponge_nl* nl) {
+    return std::max(round64(nl->stream_mean + nl->stream_mean / 5), round64(nl->stream_seen));
+}
+
+bool sa::nl_streams_seen(sponge_nl* nl, int longest) {
+    if (longest <= nl_stream_stage(nl)) return false;
+    nl->stream_seen = longest + longest / 16;
+    return true;
+}
+
 sa::PairLaunch sa::pair_launch(const sponge_nl* nl, size_t bytes_per_entry, size_t tables, int most) {
     constexpr size_t kLds = 160 * 1024, kStatic = 256;
     constexpr int kCus = 256, kWavesPerCu = 32;
     PairLaunch pl;
-    const int want = (nl->stream_mean + nl->stream_mean / 5 + 63) & ~63;
-    pl.stage = std::max(64, std::min(want, most));
+    pl.stage = std::max(64, std::min(nl_stream_stage(nl), most));
     pl.lds = pl.stage * bytes_per_entry + tables;
     pl.threads = 8 * kWave;
     if (g_recorder) return pl;
     const int most_fit = (int)(kLds / (pl.lds + kStatic));
-    const double rows = (double)nl->N / nl->G;
+    const double dense = std::max(1.0, nl->stream_seen / (1.1 * std::max(1, nl->stream_mean)));
+    const double rows = dense * nl->N / nl->G;
     double best = 0.0;
     for (int fit = 2; fit <= 6 && fit <= std::max(2, most_fit); ++fit)
         for (int split = 1; split <= 4; ++split) {
             const int waves = std::min(16, kWavesPerCu / fit);
-            const long long groups = (long long)nl->G * split;
-            const double rounds = (double)((groups + kCus * fit - 1) / (kCus * fit));
-            const double resident = std::min((double)fit, std::ceil((double)groups / kCus));
+            const double groups = nl->G * split / dense;
+            const double rounds = std::ceil(groups / (kCus * fit));
+            const double resident = std::min((double)fit, std::ceil(groups / kCus));
             const double per_simd = resident * waves / 4.0;
             const double row = std::max(5000.0, 2300.0 * per_simd);
-            const double stage = 4000.0 + 45.0 * 4.0 * nl->stream_mean / 64.0 * resident / 4.0;
+            const double stage = 4000.0 + 45.0 * 4.0 * dense * nl->stream_mean / 64.0 * resident / 4.0;
             const double cost = rounds * (stage + std::ceil(rows / (waves * split)) * row);
             if (best == 0.0 || cost < 0.97 * best) {
                 best = cost;
@@ -397,7 +412,8 @@ __device__ __forceinline__ void nl_search_cells_body(int sa_block,
     const int* __restrict__ ex_start, const int* __restrict__ ex_list,
     const int* __restrict__ ex_num, int cap, int* __restrict__ list_count,
     unsigned short* __restrict__ list, int* __restrict__ g_stream, long long* __restrict__ g_soff,
-    int* __restrict__ g_slen, unsigned long long* __restrict__ sfill, int* __restrict__ flags, float3 width, int Nx, int Ny, int Nz) {
+    int* __restrict__ g_slen, unsigned long long* __restrict__ sfill, int* __restrict__ flags, int stage,
+    float3 width, int Nx, int Ny, int Nz) {
     if (*need == 0) return;
     __shared__ float4 cand[kSearchChunk];
     __shared__ int r_first[kMaxRanges];
@@ -508,6 +524,8 @@ __device__ __forceinline__ void nl_search_cells_body(int sa_block,
         s_soff = (long long)atomicAdd(sfill, (unsigned long long)len);
         g_soff[cell] = s_soff;
         g_slen[cell] = len;
+        // flags[1]: the longest stream beyond the stage of this launch
+        if (len > stage) atomicMax(&flags[1], len);
         // running maximum of the coordinate magnitudes staged so far (only
         // grows, so each chunk's margin covers the chunk)
         s_maxbits = 0u;
@@ -718,8 +736,9 @@ __global__ void __launch_bounds__(kSearchThreads) k_nl_search_cells(
     const int* __restrict__ ex_start, const int* __restrict__ ex_list,
     const int* __restrict__ ex_num, int cap, int* __restrict__ list_count,
     unsigned short* __restrict__ list, int* __restrict__ g_stream, long long* __restrict__ g_soff,
-    int* __restrict__ g_slen, unsigned long long* __restrict__ sfill, int* __restrict__ flags, float3 width, int Nx, int Ny, int Nz) {
-    nl_search_cells_body<ORTHO>(blockIdx.x, need, spos, sexw, start, ranges, nranges, max_ranges, c, r, thr, ex_start, ex_list, ex_num, cap, list_count, list, g_stream, g_soff, g_slen, sfill, flags, width, Nx, Ny, Nz);
+    int* __restrict__ g_slen, unsigned long long* __restrict__ sfill, int* __restrict__ flags, int stage,
+    float3 width, int Nx, int Ny, int Nz) {
+    nl_search_cells_body<ORTHO>(blockIdx.x, need, spos, sexw, start, ranges, nranges, max_ranges, c, r, thr, ex_start, ex_list, ex_num, cap, list_count, list, g_stream, g_soff, g_slen, sfill, flags, stage, width, Nx, Ny, Nz);
 }
 
 
@@ -783,9 +802,10 @@ __global__ void k_nl_sum_counts(int N, const int* __restrict__ cnt, unsigned lon
 // periodic images the cells with offset in [-2, 2] (the low bound widened to
 // -3 along x / y for sheared images), sorted ascending and de-duplicated;
 // then compressed into runs of consecutive ids.  max_listed: the most cells
-// that hold one cell in their stencil (N times that bounds all streams).
+// that hold one cell in their stencil (N times that bounds all streams);
+// mean_listed: their mean.
 int build_stencil(sponge_nl* nl, std::vector<int2>& ranges, std::vector<int>& nranges,
-                  int& max_ranges, int& max_listed) {
+                  int& max_ranges, int& max_listed, double& mean_listed) {
     const int Nx = nl->Nx, Ny = nl->Ny, Nz = nl->Nz;
     const LT6 cell = nl->cell0;
     const float gl = nl->grid_length;
@@ -826,6 +846,7 @@ int build_stencil(sponge_nl* nl, std::vector<int2>& ranges, std::vector<int>& nr
         max_ranges = std::max(max_ranges, (int)rr.size());
     }
     max_listed = *std::max_element(listed.begin(), listed.end());
+    mean_listed = std::accumulate(listed.begin(), listed.end(), 0.0) / nl->G;
     ranges.assign((size_t)nl->G * max_ranges, make_int2(0, 0));
     nranges.assign(nl->G, 0);
     for (int g = 0; g < nl->G; ++g) {
@@ -933,7 +954,8 @@ extern "C" int sponge_nl_initial(sponge_nl** out, int atom_numbers, float cutoff
     std::vector<int2> ranges;
     std::vector<int> nranges;
     int max_listed = 0;
-    int rc = build_stencil(nl, ranges, nranges, nl->max_ranges, max_listed);
+    double mean_listed = 0.0;
+    int rc = build_stencil(nl, ranges, nranges, nl->max_ranges, max_listed, mean_listed);
     if (rc) {
         delete nl;
         return rc;
@@ -947,7 +969,7 @@ extern "C" int sponge_nl_initial(sponge_nl** out, int atom_numbers, float cutoff
     }
     int e = 0;
     e |= dmalloc(&nl->d_need, 1);
-    e |= dmalloc(&nl->d_flags, 1);
+    e |= dmalloc(&nl->d_flags, 2);
     e |= dmalloc(&nl->d_rebuilds, 1);
     e |= dmalloc(&nl->d_cell_count, G);
     if (own_cells) e |= dmalloc(&nl->d_ref_count, G);
@@ -974,14 +996,26 @@ extern "C" int sponge_nl_initial(sponge_nl** out, int atom_numbers, float cutoff
         return SPONGE_AMD_ERROR_MALLOC_FAILED;
     }
     {
-        // atoms within the list radius r of a cell box a x b x c at the mean
-        // density: a b c + r * surface + pi r^2 (a + b + c) + the sphere
+        // The mean stream at the box's density.  Where the search takes images
+        // nearest a cell's centre (its condition, in nl_search_cells_body): the
+        // atoms within the list radius r of a cell box a x b x c, a b c + r *
+        // surface + pi r^2 (a + b + c) + the sphere.  In other boxes (sheared
+        // cells, an axis of four cells) streams are not compacted: the atoms of
+        // the whole stencil.
         const double r = 2.0 * nl->grid_length;
-        const double a = nl->cell0.a11 / nl->Nx, b = nl->cell0.a22 / nl->Ny, d = nl->cell0.a33 / nl->Nz;
+        const float L[3] = {nl->cell0.a11, nl->cell0.a22, nl->cell0.a33};
+        const int n[3] = {nl->Nx, nl->Ny, nl->Nz};
+        const float w[3] = {nl->width.x, nl->width.y, nl->width.z};
+        bool images = nl->ortho != 0;
+        for (int k = 0; k < 3; ++k) {
+            const double edge = std::max(w[k], L[k] - (n[k] - 1) * w[k]);
+            images = images && 0.5 * L[k] > r + 0.01 + 0.5 * edge;
+        }
+        const double a = L[0] / n[0], b = L[1] / n[1], d = L[2] / n[2];
         const double reach = a * b * d + 2.0 * r * (a * b + b * d + d * a) +
                              M_PI * r * r * (a + b + d) + 4.0 / 3.0 * M_PI * r * r * r;
-        const double density = N / ((double)nl->cell0.a11 * nl->cell0.a22 * nl->cell0.a33);
-        nl->stream_mean = (int)std::min((double)N, reach * density);
+        const double mean = images ? N / ((double)L[0] * L[1] * L[2]) * reach : mean_listed * N / G;
+        nl->stream_mean = (int)std::min((double)N, mean);
     }
     hipStream_t s = nl->stream;
     hipError_t he = hipMemcpyAsync(nl->d_ranges, ranges.data(), ranges.size() * sizeof(int2),
@@ -991,7 +1025,7 @@ extern "C" int sponge_nl_initial(sponge_nl** out, int atom_numbers, float cutoff
                             hipMemcpyHostToDevice, s);
     int fe = 0;
     if (he == hipSuccess) {
-        fe |= fill_async(nl->d_flags, 0, 1, s);
+        fe |= fill_async(nl->d_flags, 0, 2, s);
         fe |= fill_async(nl->d_rebuilds, 0ull, 1, s);
         fe |= fill_async(nl->d_cell_count, 0, G, s);
         if (own_cells) fe |= fill_async(nl->d_ref_count, 0, G, s);
@@ -1108,14 +1142,14 @@ int sa::nl_update_impl(sponge_nl* nl, const int* atom_local, int local_atom_numb
                                    nl->d_nranges, nl->max_ranges, c, r, nl->thr, excluded_list_start,
                                    excluded_list, excluded_numbers, nl->cap, nl->d_list_count,
                                    nl->d_list, nl->d_stream, nl->d_soff, nl->d_slen, nl->d_sfill, nl->d_flags,
-                                   nl->width, nl->Nx, nl->Ny, nl->Nz);
+                                   nl_stream_stage(nl), nl->width, nl->Nx, nl->Ny, nl->Nz);
             } else {
                 SA_LAUNCH(kSearchThreads, (&nl_search_cells_body<true>), (k_nl_search_cells<true>), dim3(nl->G), dim3(kSearchThreads), 0, s, nl->d_need,
                                    nl->d_spos, nl->d_sexw, nl->d_cell_start, nl->d_ranges,
                                    nl->d_nranges, nl->max_ranges, c, r, nl->thr, excluded_list_start,
                                    excluded_list, excluded_numbers, nl->cap, nl->d_list_count,
                                    nl->d_list, nl->d_stream, nl->d_soff, nl->d_slen, nl->d_sfill, nl->d_flags,
-                                   nl->width, nl->Nx, nl->Ny, nl->Nz);
+                                   nl_stream_stage(nl), nl->width, nl->Nx, nl->Ny, nl->Nz);
             }
         } else {
             SA_LAUNCH(kSearchThreads, (&nl_search_cells_body<false>), (k_nl_search_cells<false>), dim3(nl->G), dim3(kSearchThreads), 0, s, nl->d_need,
@@ -1123,11 +1157,23 @@ int sa::nl_update_impl(sponge_nl* nl, const int* atom_local, int local_atom_numb
                                nl->d_nranges, nl->max_ranges, c, r, nl->thr, excluded_list_start,
                                excluded_list, excluded_numbers, nl->cap, nl->d_list_count,
                                nl->d_list, nl->d_stream, nl->d_soff, nl->d_slen, nl->d_sfill, nl->d_flags,
-                               nl->width, nl->Nx, nl->Ny, nl->Nz);
+                               nl_stream_stage(nl), nl->width, nl->Nx, nl->Ny, nl->Nz);
         }
         SA_LAUNCH_CHECK();
     }
-    nl->built = 1;
+    if (!nl->built) {
+        nl->built = 1;
+        // the first build is waited for once, so that the first force call
+        // already stages its longest stream (later ones: the overflow checks)
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (!g_recorder && hipStreamIsCapturing(s, &cs) == hipSuccess &&
+            cs == hipStreamCaptureStatusNone) {
+            int longest = 0;
+            SA_CHECK(hipMemcpyAsync(&longest, nl->d_flags + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+            SA_CHECK(hipStreamSynchronize(s));
+            nl_streams_seen(nl, longest);
+        }
+    }
     return 0;
 }
 
@@ -1148,15 +1194,17 @@ int sa::nl_set_prune(sponge_nl* nl, float delta) {
     return 0;
 }
 
-int sa::nl_take_flags(sponge_nl* nl, int* flags) {
-    int h = 0;
-    SA_CHECK(hipMemcpyAsync(&h, nl->d_flags, sizeof(int), hipMemcpyDeviceToHost, nl->stream));
+int sa::nl_take_flags(sponge_nl* nl, int* flags, bool* longer) {
+    int h[2] = {0, 0};
+    SA_CHECK(hipMemcpyAsync(h, nl->d_flags, sizeof(h), hipMemcpyDeviceToHost, nl->stream));
     SA_CHECK(hipStreamSynchronize(nl->stream));
-    if (h) {
+    if (h[0]) {
         int rc = fill_async(nl->d_flags, 0, 1, nl->stream);
         if (rc) return rc;
     }
-    *flags = h;
+    const bool grown = nl_streams_seen(nl, h[1]);
+    if (longer) *longer = grown;
+    *flags = h[0];
     return 0;
 }
 
@@ -1231,6 +1279,20 @@ extern "C" int sponge_nl_atom_group_address(sponge_nl* nl, void** d_nl) {
     if (!nl || !d_nl) return SPONGE_AMD_ERROR_VALUE_ERROR_COMMAND;
     if (!nl->d_atom_group && dmalloc(&nl->d_atom_group, nl->N)) return SPONGE_AMD_ERROR_MALLOC_FAILED;
     *d_nl = nl->d_atom_group;
+    return 0;
+}
+
+extern "C" int sponge_nl_stream_info(sponge_nl* nl, int* longest, int* staged) {
+    if (!nl) return SPONGE_AMD_ERROR_VALUE_ERROR_COMMAND;
+    if (!nl->built) return SPONGE_AMD_ERROR_MISSING_COMMAND;
+    if (longest) {
+        std::vector<int> len(nl->G);
+        SA_CHECK(hipMemcpyAsync(len.data(), nl->d_slen, sizeof(int) * nl->G, hipMemcpyDeviceToHost,
+                                nl->stream));
+        SA_CHECK(hipStreamSynchronize(nl->stream));
+        *longest = *std::max_element(len.begin(), len.end());
+    }
+    if (staged) *staged = std::min(nl_stream_stage(nl), kPairStage);
     return 0;
 }
 

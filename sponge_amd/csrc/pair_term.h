@@ -18,7 +18,6 @@ constexpr float kTwoOverSqrtPi = 1.1283791670218446f;  // Lennard_Jones_force.h:
 // polynomial erfcx, so one exponential serves erfc and the force bracket.
 // Steps that need energies or the virial use the reference's sqrtf, division
 // and erfcf.
-constexpr int kPairStage = 3584;
 constexpr int kMaxLdsTypes = 64;  // the square (A, B) table lives in LDS: up to 64 LJ types
 
 // Partner data of a row entry: from the block's LDS stage (every position of
