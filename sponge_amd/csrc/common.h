@@ -90,6 +90,29 @@ __device__ __forceinline__ float3 near_image(float3 x, float3 C, const LT6& c, c
                        x.z - c.a33 * rintf((x.z - C.z) * r.a33));
 }
 
+// A cell's centre C on one axis of the box, moved by at most 1/32 to L - k / 16
+// so that C and C - L are both exact, and the image of x nearest to it,
+// relative to it: x - C, (x - L) - C or x - (C - L), each rounded once where
+// the result is below 16 (and mostly exact), where x + L would round to the
+// box's precision (in a 35 A box that made the direct Coulomb forces an eighth
+// less exact than the minimum image's).
+__device__ __forceinline__ float image_centre(float mid, float L) {
+    return L - rintf(16.f * (L - mid)) * 0.0625f;
+}
+__device__ __forceinline__ float image_offset(float x, float C, float L, float rL) {
+    const float n = rintf((x - C) * rL);
+    return fmaf(-fmaxf(n, 0.f), L, x) - fmaf(fminf(n, 0.f), L, C);
+}
+// the distance C may be moved by, with room for rounding
+constexpr float kCentreMargin = 0.05f;
+__device__ __forceinline__ float3 image_centre(float3 mid, const LT6& c) {
+    return make_float3(image_centre(mid.x, c.a11), image_centre(mid.y, c.a22), image_centre(mid.z, c.a33));
+}
+__device__ __forceinline__ float3 image_offset(float3 x, float3 C, const LT6& c, const LT6& r) {
+    return make_float3(image_offset(x.x, C.x, c.a11, r.a11), image_offset(x.y, C.y, c.a22, r.a22),
+                       image_offset(x.z, C.z, c.a33, r.a33));
+}
+
 // r^2 as the reference's VECTOR dot product ((x*x + y*y) + z*z), no FMA.
 __device__ __forceinline__ float norm2_exact(float3 d) {
 #pragma clang fp contract(off)

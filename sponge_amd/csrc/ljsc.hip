@@ -251,7 +251,7 @@ __device__ __forceinline__ void sc_row_fast(int p, int lane, int n, const unsign
                                             unsigned short* ring) {
     const float lam = sp.lambda, lam_ = 1.0f - sp.lambda;
     const float4 pi4 = pos[p];
-    const float3 pi = near_image(make_float3(pi4.x, pi4.y, pi4.z), C, c, r);
+    const float3 pi = image_offset(make_float3(pi4.x, pi4.y, pi4.z), C, c, r);
     float fx = 0.f, fy = 0.f, fz = 0.f;
     const int npairs = (n + 1) >> 1;
     const int full = n >> 7;
@@ -371,10 +371,10 @@ __device__ __forceinline__ void ljsc_cells_body(int sa_block,
         cell_faces(ix, sg.Nx, sg.width.x, c.a11, lx, hx);
         cell_faces(iy, sg.Ny, sg.width.y, c.a22, ly, hy);
         cell_faces(iz, sg.Nz, sg.width.z, c.a33, lz, hz);
-        C = make_float3(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz));
-        shift = staged && 0.5f * c.a11 > sg.reach + 0.5f * (hx - lx) + 0.01f &&
-                0.5f * c.a22 > sg.reach + 0.5f * (hy - ly) + 0.01f &&
-                0.5f * c.a33 > sg.reach + 0.5f * (hz - lz) + 0.01f;
+        C = image_centre(make_float3(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz)), c);
+        shift = staged && 0.5f * c.a11 > sg.reach + 0.5f * (hx - lx) + kCentreMargin &&
+                0.5f * c.a22 > sg.reach + 0.5f * (hy - ly) + kCentreMargin &&
+                0.5f * c.a33 > sg.reach + 0.5f * (hz - lz) + kCentreMargin;
     }
     if (staged)
         stage_stream(
@@ -392,7 +392,7 @@ __device__ __forceinline__ void ljsc_cells_body(int sa_block,
             [&](int t, const ScStaged& e) {
                 float4 v = e.x;
                 if (shift) {
-                    const float3 im = near_image(make_float3(v.x, v.y, v.z), C, c, r);
+                    const float3 im = image_offset(make_float3(v.x, v.y, v.z), C, c, r);
                     v = make_float4(im.x, im.y, im.z, v.w);
                 }
                 cpos[t] = v;

@@ -230,23 +230,6 @@ __device__ __forceinline__ float halve16(float a, float b) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// A cell's centre C on one axis of the box, moved by at most 1/32 to L - k / 16
-// so that C and C - L are both exact, and the image of x nearest to it,
-// relative to it: x - C, (x - L) - C or x - (C - L), each rounded once where
-// the result is below 16 (and mostly exact), where x + L would round to the
-// box's precision.
-__device__ __forceinline__ float image_centre(float mid, float L) {
-    return L - rintf(16.f * (L - mid)) * 0.0625f;
-}
-__device__ __forceinline__ float image_offset(float x, float C, float L, float rL) {
-    const float n = rintf((x - C) * rL);
-    float a = x, b = C;
-    if (n >= 1.f) a = x - n * L;
-    if (n == -1.f) b = C - L;
-    if (n < -1.f) a = x - n * L;
-    return a - b;
-}
-
 // One batch of up to 64 in-range pairs added to the sums (d: displacement, q:
 // the partner's charge, 0 in lanes without a pair).
 template <bool POLY>
@@ -427,11 +410,10 @@ __global__ void __launch_bounds__(64 * kRsWaves) k_rs_features(
         cell_faces(ix, Nx, width.x, c.a11, lx, hx);
         cell_faces(iy, Ny, width.y, c.a22, ly, hy);
         cell_faces(iz, Nz, width.z, c.a33, lz, hz);
-        C = make_float3(image_centre(0.5f * (lx + hx), c.a11), image_centre(0.5f * (ly + hy), c.a22),
-                        image_centre(0.5f * (lz + hz), c.a33));
-        shift = 0.5f * c.a11 > reach + 0.5f * (hx - lx) + 0.05f &&
-                0.5f * c.a22 > reach + 0.5f * (hy - ly) + 0.05f &&
-                0.5f * c.a33 > reach + 0.5f * (hz - lz) + 0.05f;
+        C = image_centre(make_float3(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz)), c);
+        shift = 0.5f * c.a11 > reach + 0.5f * (hx - lx) + kCentreMargin &&
+                0.5f * c.a22 > reach + 0.5f * (hy - ly) + kCentreMargin &&
+                0.5f * c.a33 > reach + 0.5f * (hz - lz) + kCentreMargin;
     }
     const int* __restrict__ strm = g_stream + g_soff[cell];
     if (staged)
@@ -439,9 +421,10 @@ __global__ void __launch_bounds__(64 * kRsWaves) k_rs_features(
             strm, total, [&](int q) { return pos[q]; },
             [&](int t, const float4& v) {
                 float4 x = v;
-                if (shift)
-                    x = make_float4(image_offset(v.x, C.x, c.a11, r.a11), image_offset(v.y, C.y, c.a22, r.a22),
-                                    image_offset(v.z, C.z, c.a33, r.a33), v.w);
+                if (shift) {
+                    const float3 o = image_offset(make_float3(v.x, v.y, v.z), C, c, r);
+                    x = make_float4(o.x, o.y, o.z, v.w);
+                }
                 cpos[t] = x;
             });
     __syncthreads();
@@ -456,9 +439,7 @@ __global__ void __launch_bounds__(64 * kRsWaves) k_rs_features(
         const float4* ue = uex + sidx[p];
         const float4 x = pos[p];
         float3 pi = make_float3(x.x, x.y, x.z);
-        if (shift)
-            pi = make_float3(image_offset(x.x, C.x, c.a11, r.a11), image_offset(x.y, C.y, c.a22, r.a22),
-                             image_offset(x.z, C.z, c.a33, r.a33));
+        if (shift) pi = image_offset(pi, C, c, r);
 #define SA_RS_ROW(S, SH, P, SRC)                                                                  \
     rs_row<ORTHO, S, SH, P>(p, lane, n, row, SRC, strm, pi, c, r, rf2, inv_rf, beta, ew, ring, sums, \
                             feat, basis, ue)
