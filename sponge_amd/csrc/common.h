@@ -175,15 +175,49 @@ __device__ __forceinline__ float erfcx_poly(float x) {
     return erfcx_poly_t(__builtin_amdgcn_rcpf(1.0f + kErfcxT * x));
 }
 
-// Smooth part of the Ewald direct force factor, H(z) = (erf x - 2/sqrt(pi) x
-// e^{-x^2}) / x^3 with z = x^2: the force factor of a pair is
-// qq (1/r^3 - beta^3 H(beta^2 r^2)), with no exponential and no reciprocal
-// beside 1/r.  Polynomial of degree 12 in s = 2 z / kEwaldZMax - 1 on
-// 0 <= z <= kEwaldZMax, highest power first (error below 4e-9 in FP64 beyond
-// z = 2, and below 4e-9 of the 3 / x^3 it is subtracted from nearer; generator
-// and pins: tests/golden/make_ewald_force_fit.py, tests/test_ewald_force_fit.py).  12 fused multiply-adds against the erfcx
-// form's 8 and two quarter-rate instructions (exp2, rcp) with their
-// arguments: 14 VALU cycles less of 52 per list entry.
+// Ewald direct force bracket B(x) = erfc(x) + 2 x / sqrt(pi) exp(-x^2), x = beta
+// r: the force factor of a pair is qq B / r^3.  B = p(s)^2 with a polynomial p of
+// degree 14 in s = 2 x / kBracketXMax - 1 on 0 <= x <= kBracketXMax, highest
+// power first: neither an exponential nor a reciprocal beside 1/r, and no
+// difference of nearly equal numbers where B falls to 8e-4.  (1/r^3 minus a
+// polynomial in r^2 was 3e-4 of a pair's force off near the cutoff, against 1e-5,
+// in the same time; direct Coulomb forces of 4,143 atoms at 8 A are 4.4e-7 from
+// 64 bits, 5.9e-7 so, 4.3e-7 with the erfcx form, which takes a step of 95,000
+// atoms 2 % longer.)  Generator and pins: tests/golden/make_ewald_bracket_fit.py,
+// tests/test_ewald_bracket_fit.py.
+constexpr float kBracketXMax = 2.91547595f;
+constexpr int kBracketDegree = 14;
+constexpr float kBracket[kBracketDegree + 1] = {
+    7.479681517e-04f, 2.240266185e-04f, -3.764042864e-03f, -1.395790488e-03f, 9.287165478e-03f,
+    1.515761670e-02f, -5.182155594e-02f, -2.190603316e-02f, 2.106313556e-01f, -1.537583619e-01f,
+    -3.431663215e-01f, 5.348452926e-01f, 2.058848590e-01f, -8.598744273e-01f, 4.854928851e-01f};
+
+// B(beta r) of r.  scale = 0: beta * cutoff lies beyond the fit (an Ewald
+// tolerance below about 4e-6 at 10 A) and the callers take the erfcx form.
+struct EwaldBracket {
+    float scale;
+    __device__ __forceinline__ float operator()(float r) const {
+        const float s = fmaf(r, scale, -1.0f);
+        float p = kBracket[0];
+#pragma unroll
+        for (int k = 1; k <= kBracketDegree; ++k) p = fmaf(p, s, kBracket[k]);
+        return p * p;
+    }
+};
+
+inline EwaldBracket ewald_bracket(float beta, float cutoff) {
+    const double x = (double)beta * cutoff;
+    return {x <= (double)kBracketXMax ? (float)(2.0 * beta / (double)kBracketXMax) : 0.f};
+}
+
+// Reciprocal part of an Ewald pair's force factor, qq beta^3 H(beta^2 r^2) with
+// H(z) = (erf x - 2/sqrt(pi) x e^{-x^2}) / x^3, z = x^2 (the learned form's pair
+// field), without an exponential and with nothing to cancel at small r.
+// Polynomial of degree 12 in s = 2 z / kEwaldZMax - 1 on 0 <= z <= kEwaldZMax,
+// highest power first.  Its error in FP64 is below 9e-9 beyond z = 2 and below
+// 7e-9 of 3 / x^3 nearer (relative to H, at the splitting of a 10 A cutoff: 6e-7
+// at 1 A, 1e-6 at 0.5 A; generator and pins: tests/golden/make_ewald_force_fit.py,
+// tests/test_ewald_force_fit.py).
 constexpr float kEwaldZMax = 8.5f;
 constexpr int kEwaldDegree = 12;
 constexpr float kEwaldForce[kEwaldDegree + 1] = {
@@ -193,8 +227,7 @@ constexpr float kEwaldForce[kEwaldDegree + 1] = {
 
 // beta^3 H(beta^2 r^2) as a polynomial of r^2: beta^3 folded into the
 // coefficients, s = r^2 scale - 1.  scale = 0: beta * cutoff lies beyond the
-// fit (an Ewald tolerance below about 4e-6 at 10 A) and the callers take the
-// erfcx form.
+// fit and the caller takes erff and exp.
 struct EwaldPoly {
     float c[kEwaldDegree + 1];
     float scale;

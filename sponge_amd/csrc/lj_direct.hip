@@ -145,7 +145,7 @@ __device__ __forceinline__ void lj_row(int p, int lane, int n, const unsigned sh
                                        SRC src, const int* __restrict__ strm,
                                        const float4* __restrict__ pos, const float2* trow, int gi,
                                        const LT6& c, const LT6& r, float rc2_thr, float beta,
-                                       const EwaldPoly& ew,
+                                       EwaldBracket ew,
                                        float4* __restrict__ facc, float2* __restrict__ eacc,
                                        float* __restrict__ vacc, float3 C = float3{0.f, 0.f, 0.f},
                                        int solvent_start = 0) {
@@ -253,10 +253,10 @@ __device__ __forceinline__ void lj_row(int p, int lane, int n, const unsigned sh
 // summed into the row force by fused multiply-adds.  has = false gives the
 // absent entry of a partial pass r^2 = the cutoff threshold (out of range).
 // POLY without LJ: the row atom's charge is left to the end of the row (the
-// sums are those of q_j (beta^3 H - 1/r^3) d).
+// sums are those of -q_j B / r^3 d).
 template <bool LJ, bool POLY>
 __device__ __forceinline__ void fast_pair(const float4& pj, float2 ab, const float3& pi, float qi,
-                                          float rc2_thr, float beta, const EwaldPoly& ew, bool has,
+                                          float rc2_thr, float beta, EwaldBracket ew, bool has,
                                           float& fx, float& fy, float& fz) {
     const float3 d = make_float3(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z);
     float r2 = fmaf(d.z, d.z, fmaf(d.y, d.y, d.x * d.x));
@@ -265,7 +265,7 @@ __device__ __forceinline__ void fast_pair(const float4& pj, float2 ab, const flo
     if (POLY) {
         const float rinv = __builtin_amdgcn_rsqf(r2);
         const float ri2 = rinv * rinv;
-        const float g = fmaf(-ri2, rinv, ew(r2));
+        const float g = -(ri2 * rinv) * ew(r2 * rinv);
         if (LJ) {
             const float ri4 = ri2 * ri2;
             const float pw6 = ri4 * ri2, pw8 = ri4 * ri4;
@@ -292,7 +292,7 @@ __device__ __forceinline__ void lj_row_fast(int p, int lane, int n, const unsign
                                             const float4* cpos, const unsigned char* ctyp,
                                             const float4* __restrict__ pos, const float2* trow,
                                             const LT6& c, const LT6& r, float rc2_thr, float beta,
-                                            const EwaldPoly& ew, float4* __restrict__ facc,
+                                            EwaldBracket ew, float4* __restrict__ facc,
                                             float3 C) {
     const float4 pi4 = pos[p];
     const float3 pi = image_offset(make_float3(pi4.x, pi4.y, pi4.z), C, c, r);
@@ -369,7 +369,7 @@ __device__ __forceinline__ void lj_cells_body(int sa_block,
     const int* __restrict__ list_count, const unsigned short* __restrict__ list, int cap,
     const float4* __restrict__ pos, const int* __restrict__ ptype, const int* __restrict__ pgid,
     const float2* __restrict__ AB_sq, int T, LT6 c, LT6 r, float rc2_thr, float beta,
-    const EwaldPoly& ew, int stage, int split, float3 width, int Nx, int Ny, int Nz, float reach,
+    EwaldBracket ew, int stage, int split, float3 width, int Nx, int Ny, int Nz, float reach,
     const int* __restrict__ moved,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
     int solvent_start) {
@@ -394,7 +394,7 @@ __device__ __forceinline__ void lj_cells_body(int sa_block,
     // atom and the displacement is a plain difference, less rounded than the
     // reference's (see image_offset), and pairs beyond the cutoff stay beyond it
     // (no image is nearer than the minimum image).  Direct Coulomb forces of 4,143
-    // atoms at 8 A are 5.9e-7 from 64 bits so, 1.2e-6 with the minimum image of
+    // atoms at 8 A are 4.4e-7 from 64 bits so, 1.2e-6 with the minimum image of
     // the coordinates and 1.3e-6 with the images' own coordinates; 24,000 atoms,
     // force only, 0.3 us more for the offsets.
     float3 C = make_float3(0.f, 0.f, 0.f);
@@ -510,7 +510,7 @@ __attribute__((amdgpu_waves_per_eu(FAST && !NEED_E && !NEED_V && !SOLV ? 8 : 1))
     const int* __restrict__ list_count, const unsigned short* __restrict__ list, int cap,
     const float4* __restrict__ pos, const int* __restrict__ ptype, const int* __restrict__ pgid,
     const float2* __restrict__ AB_sq, int T, LT6 c, LT6 r, float rc2_thr, float beta,
-    EwaldPoly ew, int stage, int split, float3 width, int Nx, int Ny, int Nz, float reach,
+    EwaldBracket ew, int stage, int split, float3 width, int Nx, int Ny, int Nz, float reach,
     const int* __restrict__ moved,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
     int solvent_start) {
@@ -690,7 +690,7 @@ int launch_rows(sponge_lj* lj, sponge_nl* nl, LT6 c, LT6 r, float beta, int need
         nl, sizeof(float4) + ((need_e || need_v || solv) ? sizeof(int) : 0) + 1,
         sizeof(float2) * lj->T * lj->T + kMaxLdsTypes, lj->stage);
     const size_t sh = pl.lds;
-    const EwaldPoly ew = ewald_poly(beta, lj->cutoff);
+    const EwaldBracket ew = ewald_bracket(beta, lj->cutoff);
     const bool fast = beta * lj->cutoff <= kErfcxMax && !need_e && !need_v;
     // how far a row atom can be from its build-time cell: the automatic
     // refresh rebuilds once any atom moved more than skin * skin_permit

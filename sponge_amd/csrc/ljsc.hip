@@ -211,7 +211,7 @@ __device__ __forceinline__ unsigned short pack_types(int tp) {
 template <bool POLY>
 __device__ __forceinline__ bool sc_pair_fast(const float3& d, float r2, float qj, float2 a, float2 b,
                                              float qi, float lam, float lam_, float rc2_thr,
-                                             const ScParams& sp, const EwaldPoly& ew, bool has,
+                                             const ScParams& sp, EwaldBracket ew, bool has,
                                              float& fx, float& fy, float& fz) {
     r2 = has ? r2 : rc2_thr;
     const bool in = r2 < rc2_thr;
@@ -223,7 +223,7 @@ __device__ __forceinline__ bool sc_pair_fast(const float3& d, float r2, float qj
     const float cA = fmaf(lam, b.x, lam_ * a.x), cB = fmaf(lam, b.y, lam_ * a.y);
     float fc;
     if (POLY) {
-        fc = fmaf(r2inv, rinv, -ew(r2));
+        fc = r2inv * rinv * ew(r2 * rinv);
     } else {
         float erfc_br, bracket;
         coul_fast(r2, r2 * rinv, sp.beta, erfc_br, bracket);
@@ -246,7 +246,7 @@ __device__ __forceinline__ void sc_row_fast(int p, int lane, int n, const unsign
                                             const float4* cpos, const unsigned short* ctp,
                                             const float4* __restrict__ pos, const float2* rowA,
                                             const float2* rowB, const LT6& c, const LT6& r,
-                                            float rc2_thr, const ScParams& sp, const EwaldPoly& ew,
+                                            float rc2_thr, const ScParams& sp, EwaldBracket ew,
                                             float4* __restrict__ facc, float3 C,
                                             unsigned short* ring) {
     const float lam = sp.lambda, lam_ = 1.0f - sp.lambda;
@@ -341,7 +341,7 @@ __device__ __forceinline__ void ljsc_cells_body(int sa_block,
     const float4* __restrict__ pos, const int* __restrict__ ptp, const float* __restrict__ pqba,
     const int* __restrict__ pgid, const float2* __restrict__ ABa, int TA,
     const float2* __restrict__ ABb, int TB, LT6 c, LT6 r, float rc2_thr, ScParams sp,
-    const EwaldPoly& ew, int stage, int split,
+    EwaldBracket ew, int stage, int split,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
     double* __restrict__ du, ShiftGeom sg) {
     extern __shared__ float4 cpos[];
@@ -628,7 +628,7 @@ k_ljsc_cells(
     const int* __restrict__ list_count, const unsigned short* __restrict__ list, int cap,
     const float4* __restrict__ pos, const int* __restrict__ ptp, const float* __restrict__ pqba,
     const int* __restrict__ pgid, const float2* __restrict__ ABa, int TA,
-    const float2* __restrict__ ABb, int TB, LT6 c, LT6 r, float rc2_thr, ScParams sp, EwaldPoly ew,
+    const float2* __restrict__ ABb, int TB, LT6 c, LT6 r, float rc2_thr, ScParams sp, EwaldBracket ew,
     int stage, int split,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
     double* __restrict__ du, ShiftGeom sg) {
@@ -741,7 +741,7 @@ int launch(sponge_ljsc* h, sponge_nl* nl, LT6 c, LT6 r, float beta, bool F, bool
     const PairLaunch pl = pair_launch(
         nl, sizeof(float4) + (fast ? 0 : 2 * sizeof(int)) + sizeof(unsigned short),
         sizeof(float2) * ((size_t)h->TA * h->TA + (size_t)h->TB * h->TB) + kScRings, h->stage);
-    const EwaldPoly ew = ewald_poly(beta, h->cutoff);
+    const EwaldBracket ew = ewald_bracket(beta, h->cutoff);
     const int stage = pl.stage;
     const size_t sh = pl.lds;
 #define SA_SC(f, e, v, d, fa)                                                                      \

@@ -13,9 +13,9 @@ constexpr float kTwoOverSqrtPi = 1.1283791670218446f;  // Lennard_Jones_force.h:
 
 // Arithmetic per in-cutoff pair on force-only steps (FAST, when beta *
 // cutoff <= kErfcxMax): 1/r from the hardware rsqrt, and the Coulomb force
-// either as 1/r^3 minus the polynomial EwaldPoly (POLY, the usual Ewald
-// tolerances) or with erfc(beta r) as exp(-(beta r)^2) erfcx(beta r) with the
-// polynomial erfcx, so one exponential serves erfc and the force bracket.
+// either from the polynomial EwaldBracket (POLY, the usual Ewald tolerances) or
+// with erfc(beta r) as exp(-(beta r)^2) erfcx(beta r) with the polynomial
+// erfcx, so one exponential serves erfc and the force bracket.
 // Steps that need energies or the virial use the reference's sqrtf, division
 // and erfcf.
 constexpr int kMaxLdsTypes = 64;  // the square (A, B) table lives in LDS: up to 64 LJ types
@@ -78,7 +78,7 @@ struct PairTerm {
     float f, lx, ly, lz, elj, ec;  // f: the force factor (force = f d)
     bool in;
     __device__ __forceinline__ PairTerm(const float3& d, float r2, float qi, float qj, float2 ab,
-                                        float rc2_thr, float beta, const EwaldPoly& ew) {
+                                        float rc2_thr, float beta, EwaldBracket ew) {
         in = r2 < rc2_thr;
         // FAST: hardware rsqrt (1 ulp); otherwise the reference's sqrtf and
         // division, which energies and virials need: the LJ energy is a
@@ -99,6 +99,7 @@ struct PairTerm {
         const float qq = qi * qj;
         float erfc_br = 0.f, bracket = 0.f;
         if (FAST && POLY) {
+            bracket = ew(rabs);
         } else if (FAST) {
             coul_fast(r2, rabs, beta, erfc_br, bracket);
         } else {
@@ -107,7 +108,7 @@ struct PairTerm {
             bracket = fmaf(br * kTwoOverSqrtPi, expf(-br * br), erfc_br);
         }
         const float flj = LJ ? (ab.y - ab.x * pw6) * pw8 : 0.f;
-        const float fc = qq * (FAST && POLY ? fmaf(rinv * rinv, rinv, -ew(r2)) : pw3 * bracket);
+        const float fc = qq * pw3 * bracket;
         f = in ? flj - fc : 0.f;
         lx = f * d.x;
         ly = f * d.y;

@@ -106,7 +106,7 @@ __device__ __forceinline__ void solvent_row(
                 }
                 const float3 d = disp_pbc<ORTHO>(make_float3(xa.x, xa.y, xa.z), pb, c, r);
                 const PairTerm<false, false, FAST> t(d, norm2_exact(d), pb4.w, xa.w,
-                                                     cab[tb * T + ta], rc2_thr, beta, EwaldPoly{});
+                                                     cab[tb * T + ta], rc2_thr, beta, EwaldBracket{});
                 fb.x += t.lx;
                 fb.y += t.ly;
                 fb.z += t.lz;
@@ -122,7 +122,7 @@ __device__ __forceinline__ void solvent_row(
                                                  c, r);
                 const PairTerm<NEED_E, NEED_V, FAST> t(d, norm2_exact(d), wpos[m].w, xj.w,
                                                        cab[wtyp[m] * T + tj], rc2_thr, beta,
-                                                       EwaldPoly{});
+                                                       EwaldBracket{});
                 fw[m].x += t.lx;
                 fw[m].y += t.ly;
                 fw[m].z += t.lz;

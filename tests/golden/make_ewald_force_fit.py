@@ -1,15 +1,15 @@
-"""Generator of the Ewald force polynomial of the pair kernels' force-only path.
+"""Generator of the Ewald force polynomial of the learned form's pair field.
 
-The smooth part of the Ewald direct force,
+The reciprocal part of an Ewald pair's force,
   H(z) = (erf(x) - 2/sqrt(pi) x exp(-x^2)) / x^3,  z = x^2,
-is entire in z; the direct force factor of a pair is
-  qq (1/r^3 - beta^3 H(beta^2 r^2)),
-so it needs no exponential and no reciprocal beside 1/r.  H is fitted on
-0 <= z <= 8.5 by a polynomial of degree 12 in s = 2 z / 8.5 - 1 (in s, not z:
-the coefficients fall geometrically, so FP32 Horner evaluation stays at the
-rounding of the result).  The error is weighted by what it does to a force:
-beyond z = 2 by its absolute size, below by its size against the 1/x^3 that H
-is subtracted from (weight min(1, x^3 / 3)).  The coefficients minimise the
+is entire in z; the force factor of a pair is qq beta^3 H(beta^2 r^2), and the
+direct part is the difference to qq / r^3, so neither needs an exponential.  H
+is fitted on 0 <= z <= 8.5 by a polynomial of degree 12 in s = 2 z / 8.5 - 1 (in
+s, not z: the coefficients fall geometrically, so FP32 Horner evaluation stays
+at the rounding of the result).  The error is weighted by what it does to the
+direct force: beyond z = 2 by its absolute size, below by its size against the
+1/x^3 that H is subtracted from (weight min(1, x^3 / 3)); relative to H itself
+it is 6e-7 at x = 0.275 and 1e-6 at half of that.  The coefficients minimise the
 largest weighted error by Lawson's algorithm (iteratively reweighted least
 squares) over 4000 Chebyshev-spaced samples, in FP64 against scipy's confluent
 hypergeometric function: H(z) = 4 / (3 sqrt(pi)) 1F1(3/2; 5/2; -z).

@@ -1,4 +1,4 @@
-"""The Ewald force polynomial of the pair kernels' force-only path
+"""The Ewald force polynomial of the learned form's pair field
 (sponge_amd/csrc/common.h, kEwaldForce) against scipy, its FP32 Horner
 evaluation, and its generator (tests/golden/make_ewald_force_fit.py)
 reproducing a fit of the same accuracy."""
@@ -29,7 +29,7 @@ def committed_coefficients():
 def test_committed_constants_fp64():
     err = G.max_weighted_error(committed_coefficients()[::-1])
     print(f"FP64 max weighted error {err:.3e}")
-    assert err < 1.5e-8
+    assert err < 9e-9
 
 
 def test_committed_constants_fp32_horner():
