@@ -168,9 +168,9 @@ int sponge_nl_info(sponge_nl* nl, long long* list_entries, int* grid_dims);
 /* Candidate streams of the current list: the longest one of a cell, and how
  * many entries of a stream the pair kernels keep on chip at most (fewer where
  * LJ tables of many types take the room).  A longer stream is read from memory,
- * with the same forces.  The first sponge_nl_update waits for its build and
- * every overflow check reads the lengths since, so that the second follows the
- * first up to 3,584.  Synchronises. */
+ * with the same forces; a force call on such a list reports it, and the calls
+ * made after that one has run keep it on chip, up to 3,584 entries.
+ * Synchronises. */
 int sponge_nl_stream_info(sponge_nl* nl, int* longest, int* staged);
 
 /* Number of list builds since Initial (synchronises). */

@@ -54,7 +54,9 @@ struct sponge_nl {
     int* d_slen = nullptr;        // [G] its length
     unsigned long long* d_sfill = nullptr;  // entries of d_stream handed out in this build
     int stream_mean = 0;          // expected stream length of a cell at the mean density
-    int stream_seen = 0;          // stage for the longest stream found, where that was beyond it
+    int* h_longest = nullptr;     // pinned: a longest stream beyond the stage, stored by a pair kernel
+    int stream_seen = 0;          // stage for it
+    int stage_version = 0;        // grown so often
     int* d_exp_serial = nullptr;  // reference-format export storage (lazy)
     int* d_exp_count = nullptr;
     sa_atom_group* d_atom_group = nullptr;
@@ -183,23 +185,37 @@ constexpr int kPairStage = 3584;
 // Workgroup size and LDS of a launch of one workgroup per cell that stages the
 // cell's candidate stream (bytes per entry and of the tables beside it; at
 // most `most` entries): see its definition.
+struct StreamReport {
+    const int* longest = nullptr;  // the list's d_flags[1]
+    int* host = nullptr;           // and h_longest
+};
 struct PairLaunch {
     int stage = 0;    // entries staged; longer streams are read from HBM
     int threads = 0;
     int split = 1;    // workgroups per cell, each with every split-th group of rows
     size_t lds = 0;
+    StreamReport report;
 };
-PairLaunch pair_launch(const sponge_nl* nl, size_t bytes_per_entry, size_t tables, int most);
+PairLaunch pair_launch(sponge_nl* nl, size_t bytes_per_entry, size_t tables, int most);
 
 // Entries of a candidate stream that these launches stage, where LDS has room:
-// a fifth more than the mean expected from the box, or the longest stream that
-// a build reported with a sixteenth to spare (a stream outside the stage costs
-// its cell's rows two dependent memory reads per entry; a liquid slab in a box
-// twice as long has streams of twice the mean).  Builds report streams beyond the
-// stage (d_flags[1]); the host reads that after the first build and at every
-// overflow check and hands it to nl_streams_seen (true: the stage has grown).
+// a fifth more than the mean expected from the box, or the longest stream found
+// with a sixteenth to spare (a stream outside the stage costs its cell's rows
+// two dependent memory reads per entry; a liquid slab in a box twice as long has
+// streams of twice the mean).  The search raises d_flags[1] for streams beyond
+// the stage, the pair kernels store it to the host's word (report_streams), and
+// the host looks there before its next launch (nl_streams_poll), so that
+// nothing is waited for: the first launch on such a box reads from memory, the
+// later ones are sized for it, and a captured or recorded step is made again when
+// stage_version has moved.
 int nl_stream_stage(const sponge_nl* nl);
-bool nl_streams_seen(sponge_nl* nl, int longest);
+void nl_streams_poll(sponge_nl* nl);
+
+__device__ __forceinline__ void report_streams(const StreamReport& r, int block, int stage) {
+    if (block != 0 || threadIdx.x != 0) return;
+    const int longest = *r.longest;
+    if (longest > stage) __hip_atomic_store(r.host, longest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Lower and upper faces of cell i of n on an axis of length L (the last cell
 // ends at the box)
@@ -301,9 +317,7 @@ int md_state_arrays(sponge_md* m, float** crd, float** charge);
 int nl_set_prune(sponge_nl* nl, float delta);
 
 // the list's sticky overflow flags, read (synchronising) and cleared
-// (longer, nullable: a stream beyond the stage was found; the pair kernels'
-// launches are larger from here on)
-int nl_take_flags(sponge_nl* nl, int* flags, bool* longer = nullptr);
+int nl_take_flags(sponge_nl* nl, int* flags);
 // Check_Overflow's recovery: *nl replaced by a fresh list with 1.1x the
 // limits named by flags (the caller rebuilds anything that held the old one)
 int nl_reinitialize(sponge_nl** nl, int flags);

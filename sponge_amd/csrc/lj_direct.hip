@@ -372,12 +372,13 @@ __device__ __forceinline__ void lj_cells_body(int sa_block,
     EwaldBracket ew, int stage, int split, float3 width, int Nx, int Ny, int Nz, float reach,
     const int* __restrict__ moved,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
-    int solvent_start) {
+    int solvent_start, const StreamReport& report) {
     constexpr bool kGid = NEED_E || NEED_V || SOLV;  // global ids staged
     extern __shared__ float4 cpos[];
     int* cgid = reinterpret_cast<int*>(cpos + stage);
     float2* cab = reinterpret_cast<float2*>(cgid + (kGid ? stage : 0));
     unsigned char* ctyp = reinterpret_cast<unsigned char*>(cab + T * T);
+    report_streams(report, sa_block, stage);
     const int cell = sa_block / split, part = sa_block - cell * split;
     const int a0 = start[cell], a1 = start[cell + 1];
     if (a0 + part * (int)(blockDim.x / kWave) >= a1) return;
@@ -513,8 +514,8 @@ __attribute__((amdgpu_waves_per_eu(FAST && !NEED_E && !NEED_V && !SOLV ? 8 : 1))
     EwaldBracket ew, int stage, int split, float3 width, int Nx, int Ny, int Nz, float reach,
     const int* __restrict__ moved,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
-    int solvent_start) {
-    lj_cells_body<ORTHO, NEED_E, NEED_V, FAST, SOLV>(blockIdx.x, start, g_stream, g_soff, g_slen, list_count, list, cap, pos, ptype, pgid, AB_sq, T, c, r, rc2_thr, beta, ew, stage, split, width, Nx, Ny, Nz, reach, moved, facc, eacc, vacc, solvent_start);
+    int solvent_start, StreamReport report) {
+    lj_cells_body<ORTHO, NEED_E, NEED_V, FAST, SOLV>(blockIdx.x, start, g_stream, g_soff, g_slen, list_count, list, cap, pos, ptype, pgid, AB_sq, T, c, r, rc2_thr, beta, ew, stage, split, width, Nx, Ny, Nz, reach, moved, facc, eacc, vacc, solvent_start, report);
 }
 
 // Prune of the full rows into the inner rows that the MD driver's pair
@@ -704,7 +705,7 @@ int launch_rows(sponge_lj* lj, sponge_nl* nl, LT6 c, LT6 r, float beta, int need
                        rows_count, rows, nl->cap, lj->d_pos, lj->d_ptype, lj->d_pgid,             \
                        lj->d_AB_sq, lj->T, c, r, lj->rc2_thr, beta, ew, pl.stage, pl.split, nl->width, \
                        nl->Nx, nl->Ny, nl->Nz, reach, moved, lj->d_facc, lj->d_eacc, lj->d_vacc,  \
-                       solvent_start)
+                       solvent_start, pl.report)
 #define SA_LJ_ROWS_EVF(SV)                                      \
     if (fast) SA_LJ_ROWS(false, false, true, SV);               \
     else if (need_e && need_v) SA_LJ_ROWS(true, true, false, SV); \

@@ -343,7 +343,7 @@ __device__ __forceinline__ void ljsc_cells_body(int sa_block,
     const float2* __restrict__ ABb, int TB, LT6 c, LT6 r, float rc2_thr, ScParams sp,
     EwaldBracket ew, int stage, int split,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
-    double* __restrict__ du, ShiftGeom sg) {
+    double* __restrict__ du, ShiftGeom sg, const StreamReport& report) {
     extern __shared__ float4 cpos[];
     // force-only steps stage positions and types only (18 B per entry)
     float* cqba = reinterpret_cast<float*>(cpos + stage);
@@ -352,6 +352,7 @@ __device__ __forceinline__ void ljsc_cells_body(int sa_block,
     float2* tb = ta + TA * TA;
     unsigned short* ctp = reinterpret_cast<unsigned short*>(tb + TB * TB);
     unsigned short* ring = ctp + stage + 2 * kScRing * (threadIdx.x / kWave);
+    report_streams(report, sa_block, stage);
     const int cell = sa_block / split, part = sa_block - cell * split;
     const int a0 = start[cell], a1 = start[cell + 1];
     if (a0 + part * (int)(blockDim.x / kWave) >= a1) return;
@@ -631,10 +632,10 @@ k_ljsc_cells(
     const float2* __restrict__ ABb, int TB, LT6 c, LT6 r, float rc2_thr, ScParams sp, EwaldBracket ew,
     int stage, int split,
     float4* __restrict__ facc, float2* __restrict__ eacc, float* __restrict__ vacc,
-    double* __restrict__ du, ShiftGeom sg) {
+    double* __restrict__ du, ShiftGeom sg, StreamReport report) {
     ljsc_cells_body<ORTHO, F, E, V, DU, FAST>(blockIdx.x, start, g_stream, g_soff, g_slen,
                                          list_count, list, cap, pos, ptp, pqba, pgid, ABa, TA, ABb,
-                                         TB, c, r, rc2_thr, sp, ew, stage, split, facc, eacc, vacc, du, sg);
+                                         TB, c, r, rc2_thr, sp, ew, stage, split, facc, eacc, vacc, du, sg, report);
 }
 
 // Scatter of the rows: frc +=; atom_energy += LJ + Coulomb; the module's LJ
@@ -750,7 +751,7 @@ int launch(sponge_ljsc* h, sponge_nl* nl, LT6 c, LT6 r, float beta, bool F, bool
                        nl->d_cell_start, nl->d_stream, nl->d_soff, nl->d_slen,                      \
                        nl->d_list_count, nl->d_list, nl->cap, h->d_pos, h->d_tp, h->d_qba,          \
                        h->d_gid, h->d_ABa, h->TA, h->d_ABb, h->TB, c, r, h->rc2_thr, sp, ew, stage, pl.split, \
-                       h->d_facc, h->d_eacc, h->d_vacc, h->d_du, sg)
+                       h->d_facc, h->d_eacc, h->d_vacc, h->d_du, sg, pl.report)
     if (DU) SA_SC(false, false, false, true, false);
     else if (E && V) SA_SC(true, true, true, false, false);
     else if (E) SA_SC(true, true, false, false, false);

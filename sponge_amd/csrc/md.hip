@@ -97,6 +97,7 @@ struct sponge_md {
     // does not exist
     int* d_sx_start = nullptr;  // [N + 1]
     int* d_sx_list = nullptr;
+    int stage_version = 0;  // of the list, when steps were last captured or recorded
     int nl_generation = 0;  // bumped when recorded steps no longer hold (the list or its stage is a new one)
     float prune_delta = SPONGE_AMD_MD_LIST_PRUNE_DELTA;  // inner-row buffer of the pair kernel
     int overflow_flags = 0;  // every overflow flag seen by the driver's checks
@@ -686,18 +687,18 @@ int md_check_surrogate(sponge_md* m, long long first, long long last) {
 // step that held the old list is dropped), or is an error with
 // throw_error_when_overflow or when a cell's stream outgrew the 16-bit rows.
 int md_check_overflow(sponge_md* m, long long first, long long last) {
-    const int iv = m->nl->opt.check_overflow_interval;
-    if (iv <= 0 || (last + 1) / iv * iv < first + 1) return 0;
-    int flags = 0;
-    bool longer = false;
-    int rc = nl_take_flags(m->nl, &flags, &longer);
-    if (rc) return rc;
-    if (longer) {
+    nl_streams_poll(m->nl);
+    if (m->nl->stage_version != m->stage_version) {
         // captured and recorded steps hold the pair kernel's former stage
+        m->stage_version = m->nl->stage_version;
         drop_graphs(m);
         m->nl_generation++;
     }
-    if (!flags) return 0;
+    const int iv = m->nl->opt.check_overflow_interval;
+    if (iv <= 0 || (last + 1) / iv * iv < first + 1) return 0;
+    int flags = 0;
+    int rc = nl_take_flags(m->nl, &flags);
+    if (rc || !flags) return rc;
     m->overflow_flags |= flags;
     if ((flags & SPONGE_AMD_NL_STREAM_OVERFLOW) || m->nl->opt.throw_error_when_overflow)
         return SPONGE_AMD_ERROR_OVERFLOW;
@@ -707,6 +708,7 @@ int md_check_overflow(sponge_md* m, long long first, long long last) {
     drop_graphs(m);
     m->need_cleared = false;
     m->nl_generation++;
+    m->stage_version = 0;
     return 0;
 }
 

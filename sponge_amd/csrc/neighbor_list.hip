@@ -63,16 +63,19 @@ int sa::nl_stream_stage(const sponge_nl* nl) {
     return std::max(round64(nl->stream_mean + nl->stream_mean / 5), round64(nl->stream_seen));
 }
 
-bool sa::nl_streams_seen(sponge_nl* nl, int longest) {
-    if (longest <= nl_stream_stage(nl)) return false;
+void sa::nl_streams_poll(sponge_nl* nl) {
+    const int longest = __atomic_load_n(nl->h_longest, __ATOMIC_RELAXED);
+    if (longest <= nl_stream_stage(nl)) return;
     nl->stream_seen = longest + longest / 16;
-    return true;
+    nl->stage_version++;
 }
 
-sa::PairLaunch sa::pair_launch(const sponge_nl* nl, size_t bytes_per_entry, size_t tables, int most) {
+sa::PairLaunch sa::pair_launch(sponge_nl* nl, size_t bytes_per_entry, size_t tables, int most) {
     constexpr size_t kLds = 160 * 1024, kStatic = 256;
     constexpr int kCus = 256, kWavesPerCu = 32;
     PairLaunch pl;
+    nl_streams_poll(nl);
+    pl.report = {nl->d_flags + 1, nl->h_longest};
     pl.stage = std::max(64, std::min(nl_stream_stage(nl), most));
     pl.lds = pl.stage * bytes_per_entry + tables;
     pl.threads = 8 * kWave;
@@ -859,6 +862,8 @@ int build_stencil(sponge_nl* nl, std::vector<int2>& ranges, std::vector<int>& nr
 void nl_free(sponge_nl* nl) {
     dfree(nl->d_need);
     dfree(nl->d_flags);
+    if (nl->h_longest) (void)hipHostFree(nl->h_longest);
+    nl->h_longest = nullptr;
     dfree(nl->d_rebuilds);
     dfree(nl->d_cell_count);
     dfree(nl->d_ref_count);
@@ -970,6 +975,7 @@ extern "C" int sponge_nl_initial(sponge_nl** out, int atom_numbers, float cutoff
     int e = 0;
     e |= dmalloc(&nl->d_need, 1);
     e |= dmalloc(&nl->d_flags, 2);
+    e |= hipHostMalloc(reinterpret_cast<void**>(&nl->h_longest), sizeof(int)) != hipSuccess;
     e |= dmalloc(&nl->d_rebuilds, 1);
     e |= dmalloc(&nl->d_cell_count, G);
     if (own_cells) e |= dmalloc(&nl->d_ref_count, G);
@@ -995,6 +1001,7 @@ extern "C" int sponge_nl_initial(sponge_nl** out, int atom_numbers, float cutoff
         delete nl;
         return SPONGE_AMD_ERROR_MALLOC_FAILED;
     }
+    *nl->h_longest = 0;
     {
         // The mean stream at the box's density.  Where the search takes images
         // nearest a cell's centre (its condition, in nl_search_cells_body): the
@@ -1161,19 +1168,7 @@ int sa::nl_update_impl(sponge_nl* nl, const int* atom_local, int local_atom_numb
         }
         SA_LAUNCH_CHECK();
     }
-    if (!nl->built) {
-        nl->built = 1;
-        // the first build is waited for once, so that the first force call
-        // already stages its longest stream (later ones: the overflow checks)
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (!g_recorder && hipStreamIsCapturing(s, &cs) == hipSuccess &&
-            cs == hipStreamCaptureStatusNone) {
-            int longest = 0;
-            SA_CHECK(hipMemcpyAsync(&longest, nl->d_flags + 1, sizeof(int), hipMemcpyDeviceToHost, s));
-            SA_CHECK(hipStreamSynchronize(s));
-            nl_streams_seen(nl, longest);
-        }
-    }
+    nl->built = 1;
     return 0;
 }
 
@@ -1194,17 +1189,15 @@ int sa::nl_set_prune(sponge_nl* nl, float delta) {
     return 0;
 }
 
-int sa::nl_take_flags(sponge_nl* nl, int* flags, bool* longer) {
-    int h[2] = {0, 0};
-    SA_CHECK(hipMemcpyAsync(h, nl->d_flags, sizeof(h), hipMemcpyDeviceToHost, nl->stream));
+int sa::nl_take_flags(sponge_nl* nl, int* flags) {
+    int h = 0;
+    SA_CHECK(hipMemcpyAsync(&h, nl->d_flags, sizeof(int), hipMemcpyDeviceToHost, nl->stream));
     SA_CHECK(hipStreamSynchronize(nl->stream));
-    if (h[0]) {
+    if (h) {
         int rc = fill_async(nl->d_flags, 0, 1, nl->stream);
         if (rc) return rc;
     }
-    const bool grown = nl_streams_seen(nl, h[1]);
-    if (longer) *longer = grown;
-    *flags = h[0];
+    *flags = h;
     return 0;
 }
 
@@ -1292,6 +1285,7 @@ extern "C" int sponge_nl_stream_info(sponge_nl* nl, int* longest, int* staged) {
         SA_CHECK(hipStreamSynchronize(nl->stream));
         *longest = *std::max_element(len.begin(), len.end());
     }
+    nl_streams_poll(nl);
     if (staged) *staged = std::min(nl_stream_stage(nl), kPairStage);
     return 0;
 }

@@ -1,9 +1,9 @@
 """The stage of the pair kernels holds the streams that exist: sheared cells and
-axes of four cells (streams of the whole stencil), a liquid in a half or an
-eighth of its box (streams of twice the mean and more), from the first force
-call on; and a liquid that condenses after the first build, from the next
-overflow check on, with the same forces on both sides of it (FP64 oracle,
-test_gpu_streams.check_force)."""
+axes of four cells (streams of the whole stencil) from the start, a liquid in a
+half or an eighth of its box (streams of twice the mean and more) and one that
+condenses after the first build once a force call has met them, with the same
+forces on both sides of it (FP64 oracle, test_gpu_streams.check_force); in the
+step driver with captured steps as without."""
 import dataclasses
 
 import numpy as np
@@ -46,18 +46,37 @@ def case(name):
     return s, s.crd, abi.Box(s.box)
 
 
-@pytest.mark.parametrize("name", ["uneven", "4_cells", "elongated", "sheared", "half", "eighth"])
-def test_first_build_is_staged(dev, name):
+def force(nl, lj, d, box, beta):
     import torch
+    f = d.zeros(d.N, 3)
+    torch.cuda.synchronize()
+    lj.direct_force(nl, d.crd, d.charge, f, box, beta)
+    torch.cuda.synchronize()
+    return f.cpu().numpy()
+
+
+@pytest.mark.parametrize("name", ["uneven", "4_cells", "elongated", "sheared", "half", "eighth"])
+def test_streams_are_staged(dev, name):
+    import torch
+    from oracle import oracle as O
     from sponge_amd import abi
     s, crd, box = case(name)
     d = DevSystem(s, dev, crd)
+    beta = O.get_beta(s.cutoff, s.tolerance)
     nl = abi.NeighborList(d.N, s.cutoff, s.skin, box)
+    lj = abi.LennardJones(d.N, s.n_types, s.lj_A, s.lj_B, s.lj_type, s.cutoff)
     torch.cuda.synchronize()
     nl.update(d.crd, update=abi.NL_FORCED, excl=d.excl)
+    longest, before = nl.stream_info()
+    f = force(nl, lj, d, box, beta)
     longest, staged = nl.stream_info()
-    print(f"case: {name}: longest stream {longest}, staged {staged}", flush=True)
+    print(f"case: {name}: longest stream {longest}, staged {before}, then {staged}", flush=True)
     assert 0 < longest <= staged <= 3584
+    if name not in ("half", "eighth"):
+        assert longest <= before
+    if name != "sheared":
+        check_force(f, s)
+        check_force(force(nl, lj, d, box, beta), s)
 
 
 def test_condensing_liquid(dev):
@@ -76,18 +95,31 @@ def test_condensing_liquid(dev):
     beta = O.get_beta(s.cutoff, s.tolerance)
     torch.cuda.synchronize()
     nl.update(gas, update=abi.NL_FORCED, excl=d.excl)
+    lj.direct_force(nl, gas, d.charge, d.zeros(d.N, 3), box, beta)
     longest, staged = nl.stream_info()
     assert longest <= staged
     nl.update(d.crd, update=abi.NL_FORCED, excl=d.excl)
     longest, staged = nl.stream_info()
     assert longest > staged
-    for checked in (False, True):
-        if checked:
-            assert nl.check_overflow() == (0, 0)
-            longest, staged = nl.stream_info()
-            assert longest <= staged <= 3584
-        f = d.zeros(d.N, 3)
-        torch.cuda.synchronize()
-        lj.direct_force(nl, d.crd, d.charge, f, box, beta)
-        torch.cuda.synchronize()
-        check_force(f.cpu().numpy(), s)
+    check_force(force(nl, lj, d, box, beta), s)
+    longest, staged = nl.stream_info()
+    assert longest <= staged <= 3584
+    check_force(force(nl, lj, d, box, beta), s)
+
+
+def test_step_driver(dev):
+    import ctypes as C
+    from sponge_amd import abi
+    from sponge_amd import system as S
+    s = stretched(S.water_box(700, cutoff=8.0, seed=11), (1, 1, 2))
+    print("case: captured steps of a liquid in half of its box", flush=True)
+    eager, captured = abi.MDSystem(s), abi.MDSystem(s)
+    eager.run(41)
+    for n in (1, 20, 20):
+        captured.run(n, use_graph=True)
+    x, y = eager.state()[0], captured.state()[0]
+    assert np.abs(x.astype(np.float64) - y).max() < 1e-3
+    nl, _, _ = captured.handles()
+    longest, staged = C.c_int(), C.c_int()
+    assert captured.lib.sponge_nl_stream_info(nl, C.byref(longest), C.byref(staged)) == 0
+    assert longest.value <= staged.value
