@@ -138,7 +138,7 @@ int batch_record(sponge_batch* b) {
         sponge_pme* pme = nullptr;
         int rc = sponge_md_handles(m, &nl, &lj, &pme);
         if (!rc) pme_set_spread_waves(pme, waves);
-        if (!rc) pme_set_plane(pme, plane);
+        rec[i].plane = plane;
         if (!rc) rc = record_system(m, rec[i]);
         if (rc) return rc;
     }

@@ -110,9 +110,12 @@ struct RecordedLaunch {
 
 // lane / join_next: the recording code marks the launches that may run on a
 // side stream beside the rest of the step (lane 1), and the first launch that
-// needs their results (join_next, consumed by the next recorded launch)
+// needs their results (join_next, consumed by the next recorded launch).
+// plane: the recorded steps may transform whole planes (systems of one batch
+// take one form; the choice ends with the recording)
 struct LaunchRecorder {
     std::vector<RecordedLaunch> launches;
+    bool plane = true;
     int lane = 0;
     bool join_next = false;
 };

@@ -117,7 +117,7 @@ struct sponge_pme {
     float* d_FBCFQ = nullptr;     // [fx][fy][fz]
     float* d_BCt = nullptr;       // [fzc][fx][fy]
     double* d_acc = nullptr;      // [0] sum w BC |F|^2, [1..6] virial, [7] sum q^2, [8] sum q
-    bool plane = false;           // the x-y planes of the spectrum are transformed in LDS
+    bool plane = false;           // the x-y planes of the spectrum can be transformed in LDS
     double* d_part = nullptr;     // the convolution's partial sums of [0..6], per workgroup
     double* d_qpart = nullptr;    // the bin pass's of [7..8]
     float* d_ene = nullptr;       // [0] reciprocal, [1] self (incl. neutralizing)
@@ -282,10 +282,11 @@ hipStream_t pme_stream(const sponge_pme* p);
 bool pme_calculates_reciprocal(const sponge_pme* p);
 bool pme_updates_on(const sponge_pme* p, int step);  // the reciprocal part is evaluated this step
 void pme_set_stream(sponge_pme* p, hipStream_t s);
+// whether this step transforms the spectrum's x-y planes in LDS: the grid
+// allows it, and a recording in progress, too
+bool pme_plane(const sponge_pme* p);
 // wavefronts (tile copies) per workgroup of the tile spread, and a smaller
 // count for launches that must share one workgroup size (the batched driver)
-bool pme_plane(const sponge_pme* p);
-void pme_set_plane(sponge_pme* p, bool on);  // off for good when not on
 int pme_spread_waves(const sponge_pme* p);
 void pme_set_spread_waves(sponge_pme* p, int waves);
 int rsur_atoms(const sponge_rsur* h);

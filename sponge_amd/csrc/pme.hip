@@ -1835,7 +1835,7 @@ static int pme_fft_convolve(sponge_pme* p, int need_virial, int need_energy) {
         SA_LAUNCH_CHECK();
     }
     const ReciprocalGeom rg{p->rcell, kPI * kPI / p->beta / p->beta};
-    if (p->plane) {
+    if (pme_plane(p)) {
         const size_t sh = plane_lds(fx, fy);
         ScopedTimer timer("pme_fft_plane", s);
         if (need_energy || need_virial)
@@ -1897,9 +1897,7 @@ static int pme_fft_convolve(sponge_pme* p, int need_virial, int need_energy) {
 // spread, FFT convolution: it reads only the coordinates and charges) on a
 // stream of its own beside other work and join before the second (gather,
 // energy), which adds to the force array.  Both use the module's stream.
-bool sa::pme_plane(const sponge_pme* p) { return p->plane; }
-
-void sa::pme_set_plane(sponge_pme* p, bool on) { p->plane = p->plane && on; }
+bool sa::pme_plane(const sponge_pme* p) { return p->plane && (!g_recorder || g_recorder->plane); }
 
 int sa::pme_spread_waves(const sponge_pme* p) { return p->spread_waves; }
 
@@ -1946,7 +1944,7 @@ int sa::pme_recip_end(sponge_pme* p, const float* rcell, const float* charge, fl
         SpectrumTotals sums;
         if (need_virial || need_energy || p->opt.update_interval > 1) {
             sums.part = p->d_part;
-            sums.nx = p->plane ? p->fzc : grid_for(p->fy, p->tl_x) * p->fzc;
+            sums.nx = pme_plane(p) ? p->fzc : grid_for(p->fy, p->tl_x) * p->fzc;
             sums.acc = p->d_acc;
             sums.virial = need_virial ? d_virial : nullptr;
             if (need_energy) {
