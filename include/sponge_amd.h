@@ -379,7 +379,9 @@ int sponge_pme_update_box(sponge_pme* pme, const float* cell, const float* rcell
  * cuFFT / FFTW plans): lines per workgroup of the z, y and x passes, each the
  * fastest of {2, 4, 8, 16} by event timing of `reps` reciprocal-force calls on
  * crd / charge (device arrays) on the module's stream; chosen[3] (host, may
- * be NULL) gets the choice.  Forces do not depend on it.  Synchronises. */
+ * be NULL) gets the choice.  On a grid whose x-y planes are transformed as a
+ * whole (up to about 64 x 64) the y and x values reach no kernel and stay what
+ * they were.  Forces do not depend on it.  Synchronises. */
 int sponge_pme_autotune(sponge_pme* pme, const float* crd, const float* charge, int reps,
                         int* chosen);
 
@@ -686,8 +688,9 @@ int sponge_batch_initial(sponge_batch** out, int n_systems, sponge_md* const* sy
  * choice for systems that share a shape), then, per FFT axis, those choices
  * against one common value of {2, 4, 8, 16} timed on batched steps (one warm
  * and `reps` timed launches of 10 steps per candidate: the call advances
- * every system by 150 + 150 reps steps); tiles[3 * n_systems] (host, may be
- * NULL) gets each system's final choice.  Synchronises. */
+ * every system by 50 + 50 reps steps per axis; y and x are left out where every
+ * system transforms whole planes); tiles[3 * n_systems] (host, may be NULL)
+ * gets each system's final choice.  Synchronises. */
 int sponge_batch_autotune(sponge_batch* b, int reps, int* tiles);
 
 /* Advances every system by `steps` steps: whole launches of the graph of

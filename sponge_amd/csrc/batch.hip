@@ -313,15 +313,18 @@ int sponge_batch_autotune(sponge_batch* b, int reps, int* tiles) {
     // over the GPU); in one launch over every system longer ones may win.
     // Per axis, the per-shape choices are timed against one common value of
     // {2, 4, 8, 16} on batched steps (steps_per_launch 10: one warm launch,
-    // then `reps` timed ones), and the fastest is kept.
+    // then `reps` timed ones), and the fastest is kept.  Where every system
+    // transforms planes in LDS only the z tiling reaches a kernel.
     const size_t n = b->md.size();
     std::vector<std::array<int, 3>> cur(n), best(n);
+    bool planes = true;
     for (size_t i = 0; i < n; ++i) {
         sponge_nl* nl = nullptr;
         sponge_lj* lj = nullptr;
         sponge_pme* pme = nullptr;
         int rc = sponge_md_handles(b->md[i], &nl, &lj, &pme);
         if (rc) return rc;
+        planes = planes && pme_plane(pme);
         const auto& v = done[std::make_tuple(pme->fx, pme->fy, pme->fz)];
         cur[i] = {v[0], v[1], v[2]};
     }
@@ -348,7 +351,7 @@ int sponge_batch_autotune(sponge_batch* b, int reps, int* tiles) {
         *ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
         return rc;
     };
-    for (int a = 0; a < 3; ++a) {
+    for (int a = 0; a < (planes ? 1 : 3); ++a) {
         double best_ms = 0;
         int rc = apply(cur);
         if (!rc) rc = time_steps(&best_ms);

@@ -2086,7 +2086,8 @@ extern "C" int sponge_pme_update_box(sponge_pme* p, const float* cell, const flo
 // x passes, each chosen in turn (the others held) as the fastest of a few
 // candidates by HIP-event timing of whole reciprocal-force calls on the
 // module's stream.  Every tiling computes the same per-line transforms, so
-// forces do not depend on the choice.
+// forces do not depend on the choice.  On a grid whose planes are transformed in
+// LDS only the z tiling reaches a kernel: the other two keep their values.
 extern "C" int sponge_pme_autotune(sponge_pme* p, const float* crd, const float* charge, int reps,
                                    int* chosen) {
     if (!p || !crd || !charge || reps < 1) return SPONGE_AMD_ERROR_VALUE_ERROR_COMMAND;
@@ -2118,7 +2119,8 @@ extern "C" int sponge_pme_autotune(sponge_pme* p, const float* crd, const float*
     int* axes[3] = {&p->tl_z, &p->tl_y, &p->tl_x};
     const int cand[4] = {2, 4, 8, 16};
     rc = measure(&best_ms);
-    for (int a = 0; a < 3 && !rc; ++a) {
+    const int tuned = pme_plane(p) ? 1 : 3;
+    for (int a = 0; a < tuned && !rc; ++a) {
         const int keep = *axes[a];
         int best = keep;
         for (int c : cand) {
