@@ -1,8 +1,10 @@
 """The PME line transforms at every radix of the two-factor form (1..10, 12,
 14, 15, 16 on either side), at lengths without two factors up to 16 (125,
-162: the Stockham passes), mixed between axes, and at every tiling: the
-convolved grid and the forces against the oracle within 1e-5 relative RMS,
-reciprocal energy and virial against the FP64 oracle (gpu_helpers.
+162: the Stockham passes), mixed between axes, and at the smallest, ragged and
+largest tilings, on a grid of whole planes (where only the z tiling reaches a
+kernel), on one of two factors beyond them and on Stockham lengths on x and on
+y: the convolved grid and the forces against the oracle within 1e-5 relative
+RMS, reciprocal energy and virial against the FP64 oracle (gpu_helpers.
 check_total)."""
 import numpy as np
 import pytest
@@ -49,21 +51,28 @@ def test_grid_force_energy_virial(dev, cfg1, fft):
     check_total("virial", vir.cpu().numpy(), ref["virial"], ref64["virial"])
 
 
+@pytest.mark.parametrize("fft", [(27, 50, 125), (70, 75, 45), (125, 36, 45), (36, 125, 45)],
+                         ids=["plane", "three_passes", "stockham_x", "stockham_y"])
 @pytest.mark.parametrize("tiles", [(2, 2, 2), (4, 6, 10), (16, 16, 16), (14, 8, 12)])
-def test_tilings(dev, cfg1, tiles):
+def test_tilings(dev, cfg1, tiles, fft):
     import ctypes as C
     import torch
     from oracle import oracle as O
     from sponge_amd import abi
-    s, fft = cfg1, (27, 50, 125)
-    print(f"case: tiles {tiles}", flush=True)
-    ref = O.PME(s, fft, O.get_beta(s.cutoff, s.tolerance)).reciprocal(need_energy=False,
-                                                                      need_virial=False)
+    s = cfg1
+    print(f"case: fft {fft}, tiles {tiles}", flush=True)
+    beta = O.get_beta(s.cutoff, s.tolerance)
+    ref = O.PME(s, fft, beta).reciprocal()
+    ref64 = O.pme64(s.crd, s.charge, s.box, beta, fft)
     d = DevSystem(s, dev)
     pm = abi.ParticleMesh(d.N, abi.Box(s.box), s.cutoff, fftx=fft[0], ffty=fft[1], fftz=fft[2])
     t = (C.c_int * 3)(*tiles)
     assert pm.lib.sponge_pme_set_fft_tiling(pm.h, t) == 0
-    frc = d.zeros(d.N, 3)
-    pm.reciprocal_force(d.crd, d.charge, frc)
+    frc, plain, vir, pot = d.zeros(d.N, 3), d.zeros(d.N, 3), d.zeros(6), d.zeros(1)
+    pm.reciprocal_force(d.crd, d.charge, plain)
+    pm.reciprocal_force(d.crd, d.charge, frc, virial=vir, potential=pot)
     torch.cuda.synchronize()
+    assert rel_rms(plain.cpu().numpy(), ref["frc"]) < 1e-5
     assert rel_rms(frc.cpu().numpy(), ref["frc"]) < 1e-5
+    check_total("reciprocal", pm.step_print()["reciprocal"], ref["reciprocal"], ref64["reciprocal"])
+    check_total("virial", vir.cpu().numpy(), ref["virial"], ref64["virial"])

@@ -19,8 +19,9 @@ GRIDS = [(256, 16, 8), (16, 256, 12), (225, 20, 9), (20, 225, 10), (196, 24, 8),
          (70, 112, 16)]
 
 
-def spectrum_energy(Q, s, beta):
-    """Reciprocal energy of a charge grid in FP64."""
+def spectrum(Q, s, beta):
+    """Per point of a charge grid's spectrum, in FP64: frequencies m, m^2, the
+    squared amplitude and the influence function."""
     n, box = Q.shape, s.box.astype(np.float64)
     P = np.abs(np.fft.fftn(Q.astype(np.float64))) ** 2
     k = [np.arange(m) for m in n]
@@ -32,7 +33,31 @@ def spectrum_energy(Q, s, beta):
     bc = np.exp(-np.pi ** 2 * m2 / beta ** 2) / (np.pi * m2 * box.prod())
     bc *= b[0][:, None, None] * b[1][None, :, None] * b[2][None, None, :]
     bc[0, 0, 0] = 0.0
+    return m, m2, P, bc
+
+
+def spectrum_energy(Q, s, beta):
+    """Reciprocal energy of a charge grid."""
+    _, _, P, bc = spectrum(Q, s, beta)
     return 0.5 * (bc * P).sum()
+
+
+def spectrum_virial(Q, s, beta):
+    """Reciprocal virial (xx, xy, yy, xz, yz, zz) of a charge grid over the half
+    spectrum, its first and last planes at half weight (PM_force.cpp:1024-1068),
+    and the sums of its terms' magnitudes."""
+    m, m2, P, bc = spectrum(Q, s, beta)
+    half = Q.shape[2] // 2 + 1
+    (x, y, z), m2, P, bc = [a[:, :, :half] for a in m], *(a[:, :, :half] for a in (m2, P, bc))
+    w = np.ones(half)
+    w[0] = w[-1] = 0.5
+    f = 0.5 * w * bc * P
+    t = 2.0 / m2 * (1.0 + np.pi ** 2 / beta ** 2 * m2)
+    terms = [-f * (1 - t * x * x), f * t * x * y, -f * (1 - t * y * y), f * t * x * z,
+             f * t * y * z, -f * (1 - t * z * z)]
+    return (np.array([a.sum() for a in terms]),
+            np.array([(f * (1 + t * c)).sum() for c in (x * x, abs(x * y), y * y, abs(x * z),
+                                                         abs(y * z), z * z)]))
 
 
 @pytest.mark.parametrize("fft", GRIDS, ids=["x".join(map(str, g)) for g in GRIDS])
@@ -63,6 +88,25 @@ def test_grid_force_energy(dev, fft):
     assert rel_rms(plain.cpu().numpy(), ref["frc"]) < 1e-5
     energy = spectrum_energy(Q.cpu().numpy().reshape(fft), s, beta)
     check_total("reciprocal", pm.step_print()["reciprocal"], energy, energy)
+
+
+@pytest.mark.parametrize("fft", GRIDS, ids=["x".join(map(str, g)) for g in GRIDS])
+def test_virial(dev, fft):
+    import torch
+    from oracle import oracle as O
+    from sponge_amd import abi
+    from sponge_amd import system as S
+    s = S.config(1)
+    d = DevSystem(s, dev)
+    pm = abi.ParticleMesh(d.N, abi.Box(s.box), s.cutoff, fftx=fft[0], ffty=fft[1], fftz=fft[2])
+    frc, vir, Q = d.zeros(d.N, 3), d.zeros(6), d.zeros(int(np.prod(fft)))
+    pm.reciprocal_force(d.crd, d.charge, frc, virial=vir)
+    pm.grids(Q, None)
+    torch.cuda.synchronize()
+    want, size = spectrum_virial(Q.cpu().numpy().reshape(fft), s, O.get_beta(s.cutoff, s.tolerance))
+    e = np.abs(vir.cpu().numpy() - want) / size
+    print(f"case: fft {fft}: virial {want}, error of its terms {e.max():.2e}", flush=True)
+    assert e.max() < 1e-6
 
 
 @pytest.mark.parametrize("grids", [((28, 30, 32), (125, 28, 30)), ((28, 30, 32), (36, 25, 27))],

@@ -1,6 +1,7 @@
 """Energies and virial of the reciprocal part from the per-workgroup partial
 sums: atom counts around the bin pass's 256, each of energy and virial alone,
-and FFT tilings with the fewest and the most workgroups.  Against the FP64
+and, on a grid of the three passes, FFT tilings with the fewest and the most
+workgroups (on a grid of whole planes there is one per plane).  Against the FP64
 oracle within 1e-5 (the charge grid and its transform are FP32; a partial sum
 left out or taken twice shows at 1e-3 or more); the self and neutralizing
 energy, FP64 sums of exact FP32 products rounded once, within 1e-6."""
@@ -14,16 +15,16 @@ from gpu_helpers import DevSystem
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("fft", [(36, 40, 45), (70, 75, 45)], ids=["plane", "three_passes"])
 @pytest.mark.parametrize("n, tiles", [(1, None), (255, (2, 2, 2)), (256, (16, 16, 16)), (257, None),
                                       (1944, (4, 8, 14))])
-def test_totals(dev, n, tiles):
+def test_totals(dev, n, tiles, fft):
     import torch
     from oracle import oracle as O
     from sponge_amd import abi
     from sponge_amd import system as S
     s = S.config(1)
-    fft = (36, 40, 45)
-    print(f"case: {n} atoms, tiling {tiles}", flush=True)
+    print(f"case: {n} atoms, tiling {tiles}, fft {fft}", flush=True)
     d = DevSystem(s, dev)
     crd, charge = d.crd[:n].contiguous(), d.charge[:n].contiguous()
     pm = abi.ParticleMesh(n, abi.Box(s.box), s.cutoff, fftx=fft[0], ffty=fft[1], fftz=fft[2])
