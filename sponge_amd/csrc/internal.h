@@ -1,6 +1,7 @@
 // Module state behind the opaque handles of include/sponge_amd.h.
 #pragma once
 
+#include <memory>
 #include <vector>
 
 #include "common.h"
@@ -224,6 +225,18 @@ __device__ __forceinline__ void cell_faces(int i, int n, float width, float L, f
     hi = i == n - 1 ? L : (i + 1) * width;
 }
 
+// A stream that the step driver created.  The soft-core and learned modules it
+// drives work on it and synchronise it when they are cleared, before or after
+// the driver: each keeps the stream alive.
+struct OwnStream {
+    hipStream_t s;
+    explicit OwnStream(hipStream_t stream) : s(stream) {}
+    OwnStream(const OwnStream&) = delete;
+    OwnStream& operator=(const OwnStream&) = delete;
+    ~OwnStream() { (void)hipStreamDestroy(s); }
+};
+using StreamOwner = std::shared_ptr<OwnStream>;  // null: the caller's stream
+
 // MD-driver forms of two module calls (see their definitions)
 int lj_direct_force_md(sponge_lj* lj, sponge_nl* nl, const float* crd, const float* charge,
                        float* frc, const float* cell, const float* rcell, float pme_beta,
@@ -254,7 +267,7 @@ int rsur_features_sorted(sponge_rsur* h, sponge_nl* nl, const float4* pos, const
                          const float* charge, const float* cell, const float* rcell,
                          const int* ex_start, const int* ex_list, const int* ex_num);
 int rsur_predict_sorted(sponge_rsur* h, float* frc, int assign, const float* anchor);
-void rsur_set_stream(sponge_rsur* h, hipStream_t s);
+void rsur_set_stream(sponge_rsur* h, hipStream_t s, const StreamOwner& owner);
 // the reciprocal force in two halves (spread + FFT convolution; gather +
 // energy) on the module's stream, and that stream
 int pme_recip_begin(sponge_pme* p, const float* crd, const float* cell, const float* rcell,
@@ -297,7 +310,7 @@ int ljsc_direct_force_md(sponge_ljsc* h, sponge_nl* nl, const float* crd, const 
                          int need_atom_energy, float* atom_energy, float* atom_direct_pme_energy,
                          int* reset_flag, bool* deferred = nullptr, bool packed = false);
 const float4* ljsc_row_forces(const sponge_ljsc* h);
-void ljsc_set_stream(sponge_ljsc* h, hipStream_t s);
+void ljsc_set_stream(sponge_ljsc* h, hipStream_t s, const StreamOwner& owner);
 int ljsc_atoms(const sponge_ljsc* h);
 float ljsc_long_range_factor(const sponge_ljsc* h);
 float rsur_cutoff(const sponge_rsur* h);

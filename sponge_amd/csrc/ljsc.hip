@@ -32,6 +32,7 @@ struct sponge_ljsc {
     float lambda = 0, alpha = 0.5f, p = 1.0f, sigma6 = 729.0f, sigma6_min = 0.0f;
     float long_range_factor = 0, long_range_factor_TI = 0;
     hipStream_t stream = nullptr;
+    StreamOwner owner;             // of the stream, when it is a step driver's
     int stage = 0;                 // most stream entries staged in LDS
     float2* d_ABa = nullptr;       // [TA][TA] (A, B) of state A
     float2* d_ABb = nullptr;       // [TB][TB] of state B
@@ -1030,6 +1031,9 @@ const float4* sa::ljsc_row_forces(const sponge_ljsc* h) { return h->d_facc; }
 PackTarget sa::ljsc_pack_target(sponge_ljsc* h, const float* charge) {
     return {h->d_pos, h->d_tp, h->d_gid, charge, h->d_typeAB};
 }
-void sa::ljsc_set_stream(sponge_ljsc* h, hipStream_t s) { h->stream = s; }
+void sa::ljsc_set_stream(sponge_ljsc* h, hipStream_t s, const StreamOwner& owner) {
+    h->stream = s;
+    h->owner = owner;
+}
 int sa::ljsc_atoms(const sponge_ljsc* h) { return h->N; }
 float sa::ljsc_long_range_factor(const sponge_ljsc* h) { return h->long_range_factor; }

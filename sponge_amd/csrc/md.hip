@@ -86,7 +86,7 @@ struct sponge_md {
     double* d_sacc = nullptr;      // [0..2] sum of rec, [3] error^2, [4] reference^2, [5] last error
     unsigned long long* d_scount = nullptr;  // [0] checks, [1] fallbacks
     int use_graph = 0;
-    int own_stream = 0;  // the driver created its stream (graph capture needs one)
+    StreamOwner owner;   // of the stream, when the driver created it (graph capture needs one)
     // the reciprocal half (spread + FFT convolution) runs on a stream of its
     // own beside the list and pair work of the step, joined before the gather
     hipStream_t recip_stream = nullptr;
@@ -396,7 +396,7 @@ void md_free(sponge_md* m) {
     dfree(m->d_anchor);
     dfree(m->d_sacc);
     dfree(m->d_scount);
-    if (m->own_stream && m->stream) (void)hipStreamDestroy(m->stream);
+    m->owner.reset();  // the stream goes with its last user
     m->stream = nullptr;
     dfree(m->d_sx_start);
     dfree(m->d_sx_list);
@@ -520,7 +520,7 @@ int md_step(sponge_md* m, long long step, int need_energy, StepKind* kind_out = 
     // changes only the rounding of the total force.
     bool deferred = false;
     if (m->sc) {
-        ljsc_set_stream(m->sc, s);
+        ljsc_set_stream(m->sc, s, m->owner);
         rc = ljsc_direct_force_md(m->sc, m->nl, m->d_crd, m->d_charge, m->d_frc, cell, rcell,
                                   m->pme->beta, need_energy, m->d_atom_energy,
                                   m->pme->d_direct_atom_energy, m->nl->d_need,
@@ -742,7 +742,7 @@ extern "C" int sponge_md_initial(sponge_md** out, int atom_numbers, const float*
             delete m;
             return SPONGE_AMD_ERROR_MALLOC_FAILED;
         }
-        m->own_stream = 1;
+        m->owner = std::make_shared<OwnStream>(m->stream);
     }
     stream = m->stream;
     // default priority, like every stream of this library
@@ -1070,7 +1070,7 @@ extern "C" int sponge_md_set_surrogate(sponge_md* m, sponge_rsur* rsur, int peri
     int rc = check_surrogate(m, rsur);
     if (!rc) rc = ensure_surrogate_buffers(m);
     if (rc) return rc;
-    rsur_set_stream(rsur, m->stream);
+    rsur_set_stream(rsur, m->stream, m->owner);
     // fallbacks so far, so that only a new one switches the surrogate off
     unsigned long long cnt[2] = {0, 0};
     SA_CHECK(hipMemcpyAsync(cnt, m->d_scount, sizeof(cnt), hipMemcpyDeviceToHost, m->stream));
@@ -1117,7 +1117,7 @@ extern "C" int sponge_md_collect_frames(sponge_md* m, sponge_rsur* rsur, int n_f
     int rc = check_surrogate(m, rsur);
     if (!rc) rc = ensure_surrogate_buffers(m);
     if (rc) return rc;
-    rsur_set_stream(rsur, m->stream);
+    rsur_set_stream(rsur, m->stream, m->owner);
     // plain PME steps while collecting
     sponge_rsur* saved = m->rsur;
     m->rsur = nullptr;
@@ -1155,7 +1155,7 @@ extern "C" int sponge_md_energies(sponge_md* m, double* out) {
     SA_CHECK(hipStreamSynchronize(s));
     float lj_short = 0, lj_long = 0, pm[5] = {0, 0, 0, 0, 0};
     if (m->sc) {
-        ljsc_set_stream(m->sc, s);
+        ljsc_set_stream(m->sc, s, m->owner);
         rc = sponge_ljsc_step_print(m->sc, &lj_short);
         lj_long = ljsc_long_range_factor(m->sc) / m->volume;
     } else {

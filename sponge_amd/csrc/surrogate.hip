@@ -53,6 +53,7 @@ struct sponge_rsur {
     float rf = 0, beta = 0;
     sponge_rsur_options opt{};
     hipStream_t stream = nullptr;
+    StreamOwner owner;             // of the stream, when it is a step driver's
     int stage = 0;
     const int* sidx = nullptr;     // sorted -> local order of the last feature call's list
     const float4* pos_last = nullptr;  // sorted positions + charges the last features used
@@ -1157,7 +1158,10 @@ int rsur_predict_sorted(sponge_rsur* h, float* frc, int assign, const float* anc
     return 0;
 }
 
-void rsur_set_stream(sponge_rsur* h, hipStream_t s) { h->stream = s; }
+void rsur_set_stream(sponge_rsur* h, hipStream_t s, const StreamOwner& owner) {
+    h->stream = s;
+    h->owner = owner;
+}
 int rsur_atoms(const sponge_rsur* h) { return h->N; }
 float rsur_cutoff(const sponge_rsur* h) { return h->rf; }
 
