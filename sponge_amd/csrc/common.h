@@ -180,8 +180,8 @@ __device__ __forceinline__ float erfcx_poly(float x) {
 // degree 14 in s = 2 x / kBracketXMax - 1 on 0 <= x <= kBracketXMax, highest
 // power first: neither an exponential nor a reciprocal beside 1/r, and no
 // difference of nearly equal numbers where B falls to 8e-4.  (1/r^3 minus a
-// polynomial in r^2 was 3e-4 of a pair's force off near the cutoff, against 1e-5,
-// in the same time; direct Coulomb forces of 4,143 atoms at 8 A are 4.4e-7 from
+// polynomial in r^2 was 1.2e-4 of a pair's force off near the cutoff, against
+// 3.4e-6, in the same time; direct Coulomb forces of 4,143 atoms at 8 A are 4.4e-7 from
 // 64 bits, 5.9e-7 so, 4.3e-7 with the erfcx form, which takes a step of 95,000
 // atoms 2 % longer.)  Generator and pins: tests/golden/make_ewald_bracket_fit.py,
 // tests/test_ewald_bracket_fit.py.

@@ -1818,7 +1818,7 @@ extern "C" float* sponge_pme_direct_atom_energy(sponge_pme* p) {
     return p ? p->d_direct_atom_energy : nullptr;
 }
 
-// (the energy / virial accumulators acc[0..6] are cleared by k_pme_bin)
+// (energy and virial leave as partial sums per workgroup, which the gather adds up)
 static int pme_fft_convolve(sponge_pme* p, int need_virial, int need_energy) {
     hipStream_t s = p->stream;
     const int fx = p->fx, fy = p->fy, fz = p->fz, fzc = p->fzc;
