@@ -39,7 +39,7 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per force-only pair-kernel launch on this workload: rocprofv3
 # FETCH_SIZE and WRITE_SIZE runs scaled by a 256 MiB copy (2.0 x FETCH_SIZE,
 # 1.0 x WRITE_SIZE); commands and table in profiles/traffic_water_ions_95k.md
-PAIR_KERNEL_TRAFFIC_BYTES = 159.5e6
+PAIR_KERNEL_TRAFFIC_BYTES = 189.2e6
 # equilibration of the seeded lattice before any timed or warmup step: 100
 # steps rescaled every step, then 900 rescaled every 10 steps
 EQUIL_STEPS = 1000
