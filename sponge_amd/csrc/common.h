@@ -92,8 +92,8 @@ __device__ __forceinline__ float3 near_image(float3 x, float3 C, const LT6& c, c
 
 // A cell's centre C on one axis of the box, moved by at most 1/32 to L - k / 16
 // so that C and C - L are both exact, and the image of x nearest to it,
-// relative to it: x - C, (x - L) - C or x - (C - L), each rounded once where
-// the result is below 16 (and mostly exact), where x + L would round to the
+// relative to it: (x - n L) - C for n >= 0, (x - (n + 1) L) - (C - L) below, one
+// rounding near zero for an x inside the box, where x + L would round to the
 // box's precision (in a 35 A box that made the direct Coulomb forces an eighth
 // less exact than the minimum image's).
 __device__ __forceinline__ float image_centre(float mid, float L) {
@@ -101,7 +101,8 @@ __device__ __forceinline__ float image_centre(float mid, float L) {
 }
 __device__ __forceinline__ float image_offset(float x, float C, float L, float rL) {
     const float n = rintf((x - C) * rL);
-    return fmaf(-fmaxf(n, 0.f), L, x) - fmaf(fminf(n, 0.f), L, C);
+    const float m = __builtin_amdgcn_fmed3f(n, -1.f, 0.f);  // the box taken off C
+    return fmaf(m - n, L, x) - fmaf(m, L, C);
 }
 // the distance C may be moved by, with room for rounding
 constexpr float kCentreMargin = 0.05f;
