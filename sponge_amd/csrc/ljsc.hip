@@ -62,10 +62,11 @@ constexpr int kScStage = 3584;
 // of a plain pair), which rows near a solvated 24-atom solute met in most of
 // their passes; and 45 % of a row's list lies beyond the cutoff.
 // With the powers of lambda from the host (ScParams): force-only, 8 windows of
-// 3,600 atoms, 72 -> 54 us; energies and virial at 6,000 atoms 44 -> 36,
-// dU/dlambda 40 -> 36.  (The soft-core pairs queued for a whole workgroup,
-// 12 KB of LDS more: 83.)  What is left is the solute's own cells: all pairs of
-// a solute row are soft-core ones, five batches against one elsewhere.
+// 3,600 atoms, 72 -> 54 us (58 with displacements from the cell's centre and the
+// squared polynomial); energies and virial at 6,000 atoms 44 -> 36, dU/dlambda
+// 40 -> 36.  (The soft-core pairs queued for a whole workgroup, 12 KB of LDS
+// more: 83.)  What is left is the solute's own cells: all pairs of a solute row
+// are soft-core ones, five batches against one elsewhere.
 constexpr int kScRing = 128;
 constexpr size_t kScRings = 2 * kScRing * sizeof(unsigned short) * 16;  // of 16 wavefronts
 constexpr float kTwoOverSqrtPiF = 1.1283791670955126f;
